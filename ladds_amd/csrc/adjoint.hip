@@ -1,34 +1,41 @@
 // adjoint.hip -- hand-written adjoint of the FP64 Yoshida-4 propagation.
 //
-// Forward: the FP64 step of propagate.hip (the same acceleration<kFormFp64>), one thread
-// per object, every step of the trajectory in one launch, the state stored every K steps
-// (checkpoints).  Backward: one launch; each thread walks its checkpoint segments from the
-// last to the first, recomputes the K step-start states of a segment from its checkpoint
-// into a workspace, then runs the reverse sweep through each step:
+// Forward: the FP64 step of propagate.hip (the same acceleration<kFormFp64>), every step of
+// the trajectory in one launch, the state stored every K steps (checkpoints).
+//
+// Backward: the gradient with respect to the initial state is a product of transition
+// matrices, lambda_c = Phi_c^T lambda_{c+1}, one for each chunk of kChunk steps.  A chunk's
+// matrix depends on its first state only, so chunks are independent: one thread per (object,
+// checkpoint segment) recomputes the segment's steps from its checkpoint and carries the
+// derivative of the state with respect to the chunk's first state (6 columns) and to bc_inv
+// (a 7th) along,
 //
 //   step (v_k: velocity before kick k, r_k: position after drift k, h = dt)
-//     r_0 = r + c_0 h v_0;    v_1 = v_0 + d_0 h a(r_0, v_0, t_0)
-//     r_1 = r_0 + c_1 h v_1;  v_2 = v_1 + d_1 h a(r_1, v_1, t_1)
-//     r_2 = r_1 + c_2 h v_2;  v_3 = v_2 + d_2 h a(r_2, v_2, t_2)
-//     r'  = r_2 + c_3 h v_3;  v' = v_3
-//   reverse, with w = d_k h lambda_v:
-//     lambda_v += c_3 h lambda_r
-//     for k = 2, 1, 0:  lambda_r += J_r(r_k, v_k)^T w;  lambda_v += J_v(r_k, v_k)^T w;
-//                       lambda_bc += (da/dbc_inv) . w;  lambda_v += c_k h lambda_r
+//     r_k = r_{k-1} + c_k h v_k;   v_{k+1} = v_k + d_k h a(r_k, v_k, t_k)     k = 0, 1, 2
+//     r'  = r_2 + c_3 h v_3;       v' = v_3
+//   column (dr, dv):
+//     dr += c_k h dv;              dv += d_k h (J_r dr + J_v dv  [+ da/dbc_inv])
 //
-// The Jacobian-transpose products are derived by hand per component.  Every term except
-// drag is the gradient of a potential (Kepler, J2, C22/S22 rotated with the Earth, the
-// third bodies, cannonball SRP on the lit branch), so its Jacobian is a symmetric Hessian
-// and J^T w is the directional derivative along w.  Drag a = D rho(h) |W| W with
-// W = v - omega x r, D = -1/2 1e3 bc_inv:
-//   J_v^T w = D rho (|W| w + W (W.w)/|W|)
-//   J_r^T w = D |W| (W.w) rho'(h) r/|r| + B^T J_v^T w,  B^T u = (-omega u_y, omega u_x, 0)
-//   da/dbc_inv . w = -1/2 1e3 rho |W| (W.w)
+// and a last launch applies the transposed matrices from the last chunk to the first.  Chunks
+// begin at multiples of kChunk whatever the checkpoint spacing is, and forward and
+// recomputation evaluate the same partial accelerations (contraction fixed by the source, summed
+// in a fixed order), so the gradient does not depend on the spacing, to the last bit.  The
+// reverse sweep this replaced (recompute a segment, then walk its steps back) was one chain
+// of 8 force evaluations per step through the whole trajectory on 64 wavefronts.
+//
+// The Jacobians are derived by hand per component.  Every term except drag is the gradient
+// of a potential (Kepler, J2, C22/S22 rotated with the Earth, the third bodies, cannonball
+// SRP on the lit branch), so its part of J_r is a symmetric Hessian.  Drag
+// a = D rho(h) |W| W with W = v - omega x r = v + B r, D = -1/2 1e3 bc_inv:
+//   J_v = D rho (|W| I + W W^T/|W|)
+//   J_r = W g^T + J_v B,   g = D |W| rho'(h) r/|r|,   B = ((0, omega, 0), (-omega, 0, 0), 0)
+//   da/dbc_inv = -1/2 1e3 rho |W| W
 // Branch decisions (shadow, atmosphere row) are those of the forward trajectory: the
 // result is the derivative of the branch taken, as for any piecewise-smooth model.
 //
 // No LADDS counterpart: the reference has no differentiable propagation.  The forward
 // matches YoshidaIntegrator::integrate (OrbitPropagator @ b90f3bae, Simulation.cpp:297).
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -54,8 +61,17 @@ struct AdjointArgs {
   double *ck;             // [nck][6][n]
   const double *g_rT, *g_vT;
   double *g_r0, *g_v0, *g_bc;
-  double *work;  // [every][6][n]
+  double *phi;            // transition matrices of chunks [chunk0, chunk0 + nchunk): [nchunk][kPhi][n]
+  int chunk0, nchunk;
 };
+
+// Steps of one transition matrix: 32 make the matrices' traffic (336 bytes per object and
+// chunk) small beside the recomputation, and cut 64-step segments in two.
+constexpr int kChunk = 32;
+
+// Entries of one transition matrix: 7 columns (initial position, initial velocity, bc_inv) of
+// 6 rows (position, velocity).
+constexpr int kPhi = 42;
 
 __device__ __forceinline__ void stage_atm(AtmTable &atm) {
   const double *src = reinterpret_cast<const double *>(&c_atm_adj);
@@ -80,141 +96,223 @@ struct State {
   double x, y, z, vx, vy, vz;
 };
 
-__device__ __forceinline__ void yoshida_step(State &s, const ObjParams &p, unsigned mask, const double *cdt,
-                                             const double *ddt, const SubstepEnv<double> *env,
-                                             const AtmTable &atm) {
-  const SubstepEnv<float> unused{};
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    s.x += cdt[k] * s.vx;
-    s.y += cdt[k] * s.vy;
-    s.z += cdt[k] * s.vz;
-    double ax, ay, az;
-    acceleration<kFormFp64>(s.x, s.y, s.z, s.vx, s.vy, s.vz, p, mask, env[k], unused, atm, ax, ay, az);
-    s.vx += ddt[k] * ax;
-    s.vy += ddt[k] * ay;
-    s.vz += ddt[k] * az;
-  }
-  s.x += cdt[3] * s.vx;
-  s.y += cdt[3] * s.vy;
-  s.z += cdt[3] * s.vz;
+// Lane l's word of the environments of step s, and its store into the stage that the
+// wavefront then reads (LDS operations of a wavefront stay in order).
+__device__ __forceinline__ double fetch_env(const SubstepEnv<double> *env, int s, uint32_t lane) {
+  return lane < kEnvWords64 ? reinterpret_cast<const double *>(env + 3 * (size_t)s)[lane] : 0.0;
+}
+__device__ __forceinline__ void keep_env(SubstepEnv<double> (&stage)[3], double word, uint32_t lane) {
+  if (lane < kEnvWords64) reinterpret_cast<double *>(stage)[lane] = word;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-// Hessian-vector product of a central term f d, f = k/|d|^3, with d = sign (r - s):
-// d(d/|d|^3)/dd = (I - 3 d d^T/|d|^2)/|d|^3 and dd/dr = sign I, so
-// d/dr [f d] . w = sign f (w - 3 tau d),  tau = (d.w) / |d|^2.
-__device__ __forceinline__ void central_hvp(double dx, double dy, double dz, double f, double inv_d2, double sign,
-                                            double wx, double wy, double wz, double &gx, double &gy, double &gz) {
-  const double tau = (dx * wx + dy * wy + dz * wz) * inv_d2;
-  const double sf = sign * f;
-  gx += sf * (wx - 3.0 * tau * dx);
-  gy += sf * (wy - 3.0 * tau * dy);
-  gz += sf * (wz - 3.0 * tau * dz);
-}
+// Derivatives of the acceleration at (r, v).
+struct Jacobian {
+  double xx, xy, xz, yy, yz, zz;          // conservative part of da/dr (symmetric)
+  double d[3][3];                         // drag's part of da/dr
+  double vxx, vxy, vxz, vyy, vyz, vzz;    // da/dv (symmetric)
+  double b[3];                            // da/dbc_inv
+};
 
-// J_r^T w, J_v^T w and (da/dbc_inv).w of acceleration<kFormFp64> at (r, v).
-__device__ __forceinline__ void acceleration_vjp(double x, double y, double z, double vx, double vy, double vz,
-                                                 const ObjParams &p, unsigned mask, const SubstepEnv<double> &e,
-                                                 const AtmTable &atm, double wx, double wy, double wz, double &gx,
-                                                 double &gy, double &gz, double &gvx, double &gvy, double &gvz,
-                                                 double &gbc) {
-  const unsigned m = (p.activity == 2) ? (mask & kKepBit) : mask;
+// The four partial accelerations, with their derivatives when LIN.
+
+// Kepler, J2 and the tesseral terms: a = f r + (px, py, pz).
+template <bool LIN>
+__device__ __forceinline__ void partial_field(double x, double y, double z, unsigned mask, const SubstepEnv<double> &e,
+                                              double (&a)[3], Jacobian &o) {
+#pragma clang fp contract(on)
   const double r2 = x * x + y * y + z * z;
-  const double inv_r = rsqrt(r2);
+  const double inv_r = rsqrt64(r2);
   const double inv_r2 = inv_r * inv_r;
   const double inv_r3 = inv_r2 * inv_r;
-  const double sigma = (x * wx + y * wy + z * wz) * inv_r2;  // (r.w)/r^2
-  gx = gy = gz = gvx = gvy = gvz = gbc = 0.0;
-  if (m & kKepBit) {
-    // a = -mu r / r^3
-    const double f = -kMuEarth * inv_r3;
-    gx += f * (wx - 3.0 * sigma * x);
-    gy += f * (wy - 3.0 * sigma * y);
-    gz += f * (wz - 3.0 * sigma * z);
+  const double inv_r5 = inv_r3 * inv_r2;
+  // da/dr = d I + c r r^T + what is added to o
+  double f = 0.0, px = 0.0, py = 0.0, pz = 0.0, d = 0.0, c = 0.0;
+  if (mask & kKepBit) {
+    f = -kMuEarth * inv_r3;
+    if (LIN) {
+      d = f;
+      c = 3.0 * kMuEarth * inv_r5;
+    }
   }
-  if (m & kJ2Bit) {
-    // a = f (x (1 - z2), y (1 - z2), z (3 - z2)),  f = -kJ2Coef / r^5,  z2 = 5 z^2 / r^2
+  if (mask & kJ2Bit) {
+    // a_i = fj x_i (c_i - z2), c = (1, 1, 3), fj = -kJ2Coef/r^5, z2 = 5 z^2/r^2:
+    // da_i/dx_j = fj ((c_i - z2) delta_ij + x_i x_j/r^2 (7 z2 - 5 c_i) - 10 x_i z delta_jz/r^2)
     const double z2 = z * z * inv_r2 * 5.0;
-    const double f = -kJ2Coef * inv_r3 * inv_r2;
-    const double df = -5.0 * f * sigma;
-    const double dz2 = 10.0 * inv_r2 * z * (wz - z * sigma);
-    gx += df * x * (1.0 - z2) + f * (wx * (1.0 - z2) - x * dz2);
-    gy += df * y * (1.0 - z2) + f * (wy * (1.0 - z2) - y * dz2);
-    gz += df * z * (3.0 - z2) + f * (wz * (3.0 - z2) - z * dz2);
+    const double fj = -kJ2Coef * inv_r5;
+    const double f1 = fj * (1.0 - z2);
+    f += f1;
+    pz = 2.0 * fj * z;
+    if (LIN) {
+      const double g = fj * inv_r2;
+      const double gz = -10.0 * g * z;
+      d += f1;
+      c += g * (7.0 * z2 - 5.0);
+      o.xz += gz * x;
+      o.yz += gz * y;
+      o.zz += 2.0 * fj + 2.0 * gz * z;
+    }
   }
-  if (m & (kC22Bit | kS22Bit)) {
-    // Earth-fixed coordinates of r and w; tesseral() differentiated along w
-    const double ct = e.ct, st = e.st;
-    const double xe = ct * x + st * y, ye = -st * x + ct * y;
-    const double wxe = ct * wx + st * wy, wye = -st * wx + ct * wy;
-    const double inv_r5 = inv_r3 * inv_r2;
+  if (mask & (kC22Bit | kS22Bit)) {
+    // a = q/r^5 - 5 U r/r^7 with U = A (x^2 - y^2) + B x y, q = grad U
+    double A, B;
+    tesseral_coefficients(e, mask, A, B);
+    const double U = A * ((x - y) * (x + y)) + B * (x * y);
+    const double qx = 2.0 * A * x + B * y, qy = B * x - 2.0 * A * y;
     const double inv_r7 = inv_r5 * inv_r2;
-    double dex = 0.0, dey = 0.0, dez = 0.0;
-    if (m & kC22Bit) {
-      const double k = kC22Coef;
-      const double q = (xe * xe - ye * ye) * inv_r7 * 5.0;
-      const double dq = 10.0 * (xe * wxe - ye * wye) * inv_r7 - 7.0 * q * sigma;
-      dex += k * (2.0 * wxe * inv_r5 - 10.0 * xe * inv_r5 * sigma - wxe * q - xe * dq);
-      dey += k * (-2.0 * wye * inv_r5 + 10.0 * ye * inv_r5 * sigma - wye * q - ye * dq);
-      dez += k * (-wz * q - z * dq);
+    const double u5 = -5.0 * U * inv_r7;
+    f += u5;
+    px = qx * inv_r5;
+    py = qy * inv_r5;
+    if (LIN) {
+      const double q5 = -5.0 * inv_r7;
+      const double tx = q5 * qx, ty = q5 * qy;
+      d += u5;
+      c += -7.0 * u5 * inv_r2;
+      o.xx += 2.0 * A * inv_r5 + 2.0 * tx * x;
+      o.xy += B * inv_r5 + tx * y + ty * x;
+      o.xz += tx * z;
+      o.yy += 2.0 * ty * y - 2.0 * A * inv_r5;
+      o.yz += ty * z;
     }
-    if (m & kS22Bit) {
-      const double k = kS22Coef;
-      const double q = (xe * ye) * inv_r7 * 5.0;
-      const double dq = 5.0 * (wxe * ye + xe * wye) * inv_r7 - 7.0 * q * sigma;
-      dex += k * (wye * inv_r5 - 5.0 * ye * inv_r5 * sigma - wxe * q - xe * dq);
-      dey += k * (wxe * inv_r5 - 5.0 * xe * inv_r5 * sigma - wye * q - ye * dq);
-      dez += k * (-wz * q - z * dq);
+  }
+  a[0] = fma(f, x, px);
+  a[1] = fma(f, y, py);
+  a[2] = fma(f, z, pz);
+  if (LIN) {
+    const double cx = c * x, cy = c * y, cz = c * z;
+    o.xx += cx * x + d;
+    o.xy += cx * y;
+    o.xz += cx * z;
+    o.yy += cy * y + d;
+    o.yz += cy * z;
+    o.zz += cz * z + d;
+  }
+}
+
+// a = al W, al = D rho |W|.
+template <bool LIN>
+__device__ __forceinline__ void partial_drag(double x, double y, double z, double vx, double vy, double vz,
+                                             double drag64, const AtmTable &atm, double (&a)[3], Jacobian &o) {
+#pragma clang fp contract(on)
+  const double om = kOmegaEarth;
+  const double wx = vx + om * y, wy = vy - om * x, wz = vz;
+  const double w2 = wx * wx + wy * wy + wz * wz;
+  const double inv_w = rsqrt64(fmax(w2, 1e-290));
+  const double wn = w2 * inv_w;  // 0 without wind
+  const double r2 = x * x + y * y + z * z;
+  const double inv_r = rsqrt64(r2);
+  const double h = r2 * inv_r - kREarth;
+  const AtmRow &row = atm_row(h, atm);
+  const double inv_scale = row.inv_scale;
+  const double rho = row.rho * exp64((row.h0 - h) * inv_scale);
+  const double dr = drag64 * rho;
+  const double al = dr * wn;
+  a[0] = al * wx;
+  a[1] = al * wy;
+  a[2] = al * wz;
+  if (LIN) {
+    const double s = dr * (w2 > 0.0 ? inv_w : 0.0);
+    const double sx = s * wx, sy = s * wy, sz = s * wz;
+    o.vxx = sx * wx + al;
+    o.vxy = sx * wy;
+    o.vxz = sx * wz;
+    o.vyy = sy * wy + al;
+    o.vyz = sy * wz;
+    o.vzz = sz * wz + al;
+    const double bw = kDragCoef * rho * wn;
+    o.b[0] = bw * wx;
+    o.b[1] = bw * wy;
+    o.b[2] = bw * wz;
+    const double gr = -al * inv_scale * inv_r;
+    const double gx = gr * x, gy = gr * y, gz = gr * z;
+    o.d[0][0] = wx * gx - om * o.vxy;
+    o.d[0][1] = wx * gy + om * o.vxx;
+    o.d[0][2] = wx * gz;
+    o.d[1][0] = wy * gx - om * o.vyy;
+    o.d[1][1] = wy * gy + om * o.vxy;
+    o.d[1][2] = wy * gz;
+    o.d[2][0] = wz * gx - om * o.vyz;
+    o.d[2][1] = wz * gy + om * o.vxz;
+    o.d[2][2] = wz * gz;
+  }
+}
+
+// Central term k d/|d|^3, d = s - r, less the indirect term; its Hessian is
+// -k/|d|^3 (I - 3 d d^T/|d|^2).
+template <bool LIN>
+__device__ __forceinline__ void partial_central(double x, double y, double z, const double *s, double k,
+                                                const double *indirect, bool gravity, double (&a)[3], Jacobian &o) {
+#pragma clang fp contract(on)
+  const double dx = s[0] - x, dy = s[1] - y, dz = s[2] - z;
+  const double inv_d = rsqrt64(dx * dx + dy * dy + dz * dz);
+  const double inv_d2 = inv_d * inv_d;
+  const double f = k * (inv_d2 * inv_d);
+  const double go = gravity ? 1.0 : 0.0;
+  a[0] = fma(f, dx, -go * indirect[0]);
+  a[1] = fma(f, dy, -go * indirect[1]);
+  a[2] = fma(f, dz, -go * indirect[2]);
+  if (LIN) {
+    const double c = 3.0 * f * inv_d2;
+    const double cx = c * dx, cy = c * dy, cz = c * dz;
+    o.xx += cx * dx - f;
+    o.xy += cx * dy;
+    o.xz += cx * dz;
+    o.yy += cy * dy - f;
+    o.yz += cy * dz;
+    o.zz += cz * dz - f;
+  }
+}
+
+// Partial acceleration `group` (0: Earth's field, 1: drag, 2: Sun and SRP, 3: Moon); zero
+// where its components are off.
+template <bool LIN>
+__device__ __forceinline__ void partial_acceleration(int group, const State &s, const ObjParams &p, unsigned mask,
+                                                     const SubstepEnv<double> &e, const AtmTable &atm,
+                                                     double (&a)[3], Jacobian &o) {
+#pragma clang fp contract(on)
+  a[0] = a[1] = a[2] = 0.0;
+  if (group == 0) {
+    if (mask & (kKepBit | kJ2Bit | kC22Bit | kS22Bit)) partial_field<LIN>(s.x, s.y, s.z, mask, e, a, o);
+  } else if (group == 1) {
+    if (mask & kDragBit) partial_drag<LIN>(s.x, s.y, s.z, s.vx, s.vy, s.vz, p.drag64, atm, a, o);
+  } else if (group == 2) {
+    if (mask & (kSolBit | kSrpBit)) {
+      double k = (mask & kSolBit) ? kGmSun : 0.0;
+      const double r2 = s.x * s.x + s.y * s.y + s.z * s.z;
+      if (mask & kSrpBit) k -= in_shadow(s.x, s.y, s.z, r2, e) ? 0.0 : p.srp64;
+      partial_central<LIN>(s.x, s.y, s.z, e.sun, k, e.sun_acc, (mask & kSolBit) != 0, a, o);
     }
-    gx += ct * dex - st * dey;
-    gy += st * dex + ct * dey;
-    gz += dez;
+  } else {
+    if (mask & kLunBit) partial_central<LIN>(s.x, s.y, s.z, e.moon, kGmMoon, e.moon_acc, true, a, o);
   }
-  if (m & kSolBit) {
-    // a += GM d/|d|^3 with d = s - r (the indirect term does not depend on r)
-    const double dx = e.sun[0] - x, dy = e.sun[1] - y, dz = e.sun[2] - z;
-    const double inv_d2 = 1.0 / (dx * dx + dy * dy + dz * dz);
-    const double inv_d = sqrt(inv_d2);
-    central_hvp(dx, dy, dz, kGmSun * inv_d2 * inv_d, inv_d2, -1.0, wx, wy, wz, gx, gy, gz);
+}
+
+// The sum of the four, in the order of the forward's exchange.
+template <bool LIN>
+__device__ __forceinline__ void total_acceleration(const State &s, const ObjParams &p, unsigned mask,
+                                                   const SubstepEnv<double> &e, const AtmTable &atm, double (&a)[3],
+                                                   Jacobian &o) {
+  double b[3];
+  partial_acceleration<LIN>(0, s, p, mask, e, atm, a, o);
+#pragma unroll
+  for (int g = 1; g < 4; ++g) {
+    partial_acceleration<LIN>(g, s, p, mask, e, atm, b, o);
+    for (int q = 0; q < 3; ++q) a[q] += b[q];
   }
-  if (m & kLunBit) {
-    const double dx = e.moon[0] - x, dy = e.moon[1] - y, dz = e.moon[2] - z;
-    const double inv_d2 = 1.0 / (dx * dx + dy * dy + dz * dz);
-    const double inv_d = sqrt(inv_d2);
-    central_hvp(dx, dy, dz, kGmMoon * inv_d2 * inv_d, inv_d2, -1.0, wx, wy, wz, gx, gy, gz);
-  }
-  if ((m & kSrpBit) && !in_shadow(x, y, z, r2, e)) {
-    // a += srp d/|d|^3 with d = r - s
-    const double dx = x - e.sun[0], dy = y - e.sun[1], dz = z - e.sun[2];
-    const double inv_d2 = 1.0 / (dx * dx + dy * dy + dz * dz);
-    const double inv_d = sqrt(inv_d2);
-    central_hvp(dx, dy, dz, p.srp64 * inv_d2 * inv_d, inv_d2, 1.0, wx, wy, wz, gx, gy, gz);
-  }
-  if (m & kDragBit) {
-    const double om = kOmegaEarth;
-    const double Wx = vx + om * y, Wy = vy - om * x, Wz = vz;
-    const double vn = sqrt(Wx * Wx + Wy * Wy + Wz * Wz);
-    const double h = r2 * inv_r - kREarth;
-    const int row = atm_row(h, atm);
-    const double rho = atm.rho[row] * exp(-(h - atm.h0[row]) * atm.inv_scale[row]);
-    const double drho = -rho * atm.inv_scale[row];
-    const double Ww = Wx * wx + Wy * wy + Wz * wz;
-    const double D = p.drag64;
-    // J_v^T w
-    const double inv_vn = vn > 0.0 ? 1.0 / vn : 0.0;
-    const double jvx = D * rho * (vn * wx + Wx * Ww * inv_vn);
-    const double jvy = D * rho * (vn * wy + Wy * Ww * inv_vn);
-    const double jvz = D * rho * (vn * wz + Wz * Ww * inv_vn);
-    gvx += jvx;
-    gvy += jvy;
-    gvz += jvz;
-    // J_r^T w: density gradient along r/|r| plus the co-rotation term B^T J_v^T w
-    const double fr = D * vn * Ww * drho * inv_r;
-    gx += fr * x - om * jvy;
-    gy += fr * y + om * jvx;
-    gz += fr * z;
-    gbc += kDragCoef * rho * vn * Ww;
-  }
+}
+
+// Drift and kick of the composition, contracted the same way everywhere.
+__device__ __forceinline__ void drift(State &s, double cdt) {
+  s.x = fma(cdt, s.vx, s.x);
+  s.y = fma(cdt, s.vy, s.y);
+  s.z = fma(cdt, s.vz, s.z);
+}
+__device__ __forceinline__ void kick(State &s, double ddt, const double (&a)[3]) {
+  s.vx = fma(ddt, a[0], s.vx);
+  s.vy = fma(ddt, a[1], s.vy);
+  s.vz = fma(ddt, a[2], s.vz);
 }
 
 __device__ __forceinline__ void load_state(State &s, const double *base, size_t n, size_t i) {
@@ -235,91 +333,75 @@ __device__ __forceinline__ void store_state(const State &s, double *base, size_t
   base[5 * n + i] = s.vz;
 }
 
-// Four wavefronts per workgroup share 64 objects: wavefront w evaluates the component
-// group kGroupMask[w] of every acceleration (and of its adjoint) for the 64 objects, the
-// four partial results are summed through LDS in a fixed order, and every wavefront then
-// carries the same integrator state.  One object's force evaluation is thus spread over
-// the four SIMDs of a CU (the sweep over steps is sequential, so this is where the
-// parallelism is).  Groups are balanced by cost.
+// The forward pass is one chain of steps.  Up to kGroupObjects objects (half a wavefront per
+// SIMD at one thread per object) four wavefronts share 64 objects: wavefront w evaluates
+// partial acceleration w, the four are summed through LDS, and every wavefront then carries
+// the same integrator state.  With more objects one thread per object fills the SIMDs without
+// the exchange.
 constexpr int kAdjWaves = 4;
 constexpr int kAdjLanes = 64;
-__device__ constexpr unsigned kGroupMask[kAdjWaves] = {kKepBit | kJ2Bit | kSrpBit, kDragBit, kC22Bit | kS22Bit,
-                                                       kSolBit | kLunBit};
+constexpr size_t kGroupObjects = 32768;
 
-// Partial sums of the four wavefronts, double-buffered so that one barrier per exchange
-// suffices: a buffer is rewritten only after the next exchange's barrier, which every
-// wavefront reaches after reading it.
-struct GroupExchange {
-  double buf[2][kAdjWaves][8][kAdjLanes];
-  int parity;
-};
-
-template <int NV>
-__device__ __forceinline__ void group_sum(GroupExchange &x, int &parity, double (&v)[NV]) {
-  const int w = threadIdx.x / kAdjLanes, l = threadIdx.x % kAdjLanes;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) x.buf[parity][w][k][l] = v[k];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-    v[k] = ((x.buf[parity][0][k][l] + x.buf[parity][1][k][l]) + x.buf[parity][2][k][l]) + x.buf[parity][3][k][l];
-  parity ^= 1;
+// Dummies keep their state; evasivePreserving objects feel the Keplerian term only.
+__device__ __forceinline__ unsigned object_mask(const ObjParams &p, unsigned mask) {
+  return p.activity == 2 ? mask & kKepBit : mask;
 }
 
-__device__ __forceinline__ void group_acceleration(const State &s, const ObjParams &p, unsigned gmask,
-                                                   const SubstepEnv<double> &env, const AtmTable &atm,
-                                                   GroupExchange &x, int &parity, double &ax, double &ay,
-                                                   double &az) {
-  const SubstepEnv<float> unused{};
-  double v[3];
-  acceleration<kFormFp64>(s.x, s.y, s.z, s.vx, s.vy, s.vz, p, gmask, env, unused, atm, v[0], v[1], v[2]);
-  group_sum<3>(x, parity, v);
-  ax = v[0];
-  ay = v[1];
-  az = v[2];
-}
-
-// One Yoshida step (the composition of propagate.hip) with group-split accelerations;
-// `moving` false keeps the state (dummies) while the wavefront still takes part in the
-// exchanges.
-__device__ __forceinline__ void group_step(State &s, const ObjParams &p, unsigned gmask, bool moving,
-                                           const double *cdt, const double *ddt, const SubstepEnv<double> *env,
-                                           const AtmTable &atm, GroupExchange &x, int &parity) {
-  const double go = moving ? 1.0 : 0.0;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    s.x += go * cdt[k] * s.vx;
-    s.y += go * cdt[k] * s.vy;
-    s.z += go * cdt[k] * s.vz;
-    double ax, ay, az;
-    group_acceleration(s, p, gmask, env[k], atm, x, parity, ax, ay, az);
-    s.vx += go * ddt[k] * ax;
-    s.vy += go * ddt[k] * ay;
-    s.vz += go * ddt[k] * az;
-  }
-  s.x += go * cdt[3] * s.vx;
-  s.y += go * cdt[3] * s.vy;
-  s.z += go * cdt[3] * s.vz;
-}
-
-__global__ __launch_bounds__(kAdjWaves * kAdjLanes) void k_adjoint_forward(AdjointArgs a) {
+template <bool GROUPED>
+__global__ __launch_bounds__(kAdjWaves *kAdjLanes) void k_adjoint_forward(AdjointArgs a) {
   __shared__ AtmTable atm;
-  __shared__ GroupExchange x;
+  // partial sums of the four wavefronts, double-buffered: one barrier per exchange, since a
+  // buffer is rewritten only after the next exchange's barrier, which every wavefront reaches
+  // after reading it
+  __shared__ double part[GROUPED ? 2 : 1][GROUPED ? kAdjWaves : 1][3][kAdjLanes];
+  __shared__ SubstepEnv<double> stage[kAdjWaves][2][3];
   stage_atm(atm);
-  const int w = threadIdx.x / kAdjLanes, l = threadIdx.x % kAdjLanes;
-  const size_t n = a.n, i = (size_t)blockIdx.x * kAdjLanes + l;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kAdjLanes));
+  const uint32_t l = threadIdx.x % kAdjLanes;
+  const size_t n = a.n, i = (GROUPED ? (size_t)blockIdx.x : (size_t)blockIdx.x * kAdjWaves + w) * kAdjLanes + l;
   const bool live = i < n;
   const size_t ii = live ? i : 0;  // lanes past the end compute on object 0 and write nothing
+  const bool writes = live && (!GROUPED || w == 0);
   State s{a.r0[ii], a.r0[n + ii], a.r0[2 * n + ii], a.v0[ii], a.v0[n + ii], a.v0[2 * n + ii]};
   const ObjParams p = object_params(a, ii);
-  const bool moving = p.activity >= 0;  // dummies keep their state
-  const unsigned gmask = a.mask & kGroupMask[w];
-  int parity = 0;
+  const unsigned mask = object_mask(p, a.mask);
+  const bool moving = p.activity >= 0;
+  Jacobian unused;
+  int parity = 0, until = 0;  // until: steps to the next checkpoint
+  double next = fetch_env(a.env, 0, l);
+  keep_env(stage[w][0], next, l);
+  double *ck = a.ck;
   for (int step = 0; step < a.nsteps; ++step) {
-    if (w == 0 && live && step % a.every == 0) store_state(s, a.ck + (size_t)(step / a.every) * 6 * n, n, i);
-    group_step(s, p, gmask, moving, a.cdt, a.ddt, a.env + 3 * step, atm, x, parity);
+    if (until == 0) {
+      if (writes) store_state(s, ck, n, i);
+      ck += 6 * n;
+      until = a.every;
+    }
+    until -= 1;
+    if (step + 1 < a.nsteps) next = fetch_env(a.env, step + 1, l);
+    const SubstepEnv<double> *env = stage[w][step & 1];
+    State t = s;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      drift(t, a.cdt[k]);
+      double acc[3];
+      if constexpr (GROUPED) {
+        partial_acceleration<false>(w, t, p, mask, env[k], atm, acc, unused);
+        for (int q = 0; q < 3; ++q) part[parity][w][q][l] = acc[q];
+        __syncthreads();
+        for (int q = 0; q < 3; ++q)
+          acc[q] = ((part[parity][0][q][l] + part[parity][1][q][l]) + part[parity][2][q][l]) + part[parity][3][q][l];
+        parity ^= 1;
+      } else {
+        total_acceleration<false>(t, p, mask, env[k], atm, acc, unused);
+      }
+      kick(t, a.ddt[k], acc);
+    }
+    drift(t, a.cdt[3]);
+    if (moving) s = t;
+    if (step + 1 < a.nsteps) keep_env(stage[w][(step + 1) & 1], next, l);
   }
-  if (w == 0 && live) {
+  if (writes) {
     a.rT[i] = s.x;
     a.rT[n + i] = s.y;
     a.rT[2 * n + i] = s.z;
@@ -329,93 +411,147 @@ __global__ __launch_bounds__(kAdjWaves * kAdjLanes) void k_adjoint_forward(Adjoi
   }
 }
 
-__global__ __launch_bounds__(kAdjWaves * kAdjLanes) void k_adjoint_backward(AdjointArgs a) {
+// Transition matrices for 64 objects: of the chunks of [a.chunk0, a.chunk0 + a.nchunk) that
+// begin in one checkpoint segment, or (segments shorter than a chunk) of one chunk.
+__global__ __launch_bounds__(kAdjLanes) __attribute__((amdgpu_waves_per_eu(2)))
+void k_adjoint_segments(AdjointArgs a) {
   __shared__ AtmTable atm;
-  __shared__ GroupExchange x;
+  __shared__ SubstepEnv<double> stage[2][3];
   stage_atm(atm);
-  const int w = threadIdx.x / kAdjLanes, l = threadIdx.x % kAdjLanes;
+  const uint32_t l = threadIdx.x;
   const size_t n = a.n, i = (size_t)blockIdx.x * kAdjLanes + l;
   const bool live = i < n;
   const size_t ii = live ? i : 0;
-  double lx = a.g_rT ? a.g_rT[ii] : 0.0, ly = a.g_rT ? a.g_rT[n + ii] : 0.0, lz = a.g_rT ? a.g_rT[2 * n + ii] : 0.0;
-  double lvx = a.g_vT ? a.g_vT[ii] : 0.0, lvy = a.g_vT ? a.g_vT[n + ii] : 0.0,
-         lvz = a.g_vT ? a.g_vT[2 * n + ii] : 0.0;
-  double lbc = 0.0;
+  int seg, first, last;  // chunks [first, last) from the checkpoint of segment seg
+  if (a.every < kChunk) {
+    first = a.chunk0 + (int)blockIdx.y;
+    last = first + 1;
+    seg = first * kChunk / a.every;
+  } else {
+    seg = a.chunk0 * kChunk / a.every + (int)blockIdx.y;
+    first = max(a.chunk0, (seg * a.every + kChunk - 1) / kChunk);
+    last = min(a.chunk0 + a.nchunk, (min((seg + 1) * a.every, a.nsteps) + kChunk - 1) / kChunk);
+  }
+  if (first >= last) return;
+  State s;
+  load_state(s, a.ck + (size_t)seg * 6 * n, n, ii);
   const ObjParams p = object_params(a, ii);
-  const bool moving = p.activity >= 0;
-  const unsigned gmask = a.mask & kGroupMask[w];
-  int parity = 0;
-  for (int seg = a.nck - 1; seg >= 0; --seg) {
-    const int s0 = seg * a.every;
-    const int s1 = min(s0 + a.every, a.nsteps);
-    // Recompute the step-start states of the segment.  Every wavefront holds the same
-    // values (same operations on the same inputs) and stores them to the same addresses,
-    // so each thread reads back exactly what it wrote.
-    State s;
-    load_state(s, a.ck + (size_t)seg * 6 * n, n, ii);
-    for (int step = s0; step < s1; ++step) {
-      if (live) store_state(s, a.work + (size_t)(step - s0) * 6 * n, n, i);
-      if (step + 1 < s1) group_step(s, p, gmask, moving, a.cdt, a.ddt, a.env + 3 * step, atm, x, parity);
+  const unsigned mask = object_mask(p, a.mask);
+  int step = seg * a.every;
+  const int end = min(last * kChunk, a.nsteps);
+  double next = fetch_env(a.env, step, l);
+  keep_env(stage[step & 1], next, l);
+  // to the first chunk
+  for (; step < first * kChunk; ++step) {
+    next = fetch_env(a.env, step + 1, l);
+#pragma unroll 1
+    for (int k = 0; k < 3; ++k) {
+      drift(s, a.cdt[k]);
+      double acc[3];
+      Jacobian unused;
+      total_acceleration<false>(s, p, mask, stage[step & 1][k], atm, acc, unused);
+      kick(s, a.ddt[k], acc);
     }
-    for (int step = s1 - 1; step >= s0; --step) {
-      if (live) load_state(s, a.work + (size_t)(step - s0) * 6 * n, n, i);
-      const SubstepEnv<double> *env = a.env + 3 * step;
-      // forward through the step, keeping the kick inputs (r_k, v_k)
-      double rx[3], ry[3], rz[3], ux[3], uy[3], uz[3];
+    drift(s, a.cdt[3]);
+    keep_env(stage[(step + 1) & 1], next, l);
+  }
+  double R[7][3], V[7][3];
+#pragma unroll 1
+  for (int chunk = first; chunk < last; ++chunk) {
 #pragma unroll
+    for (int c = 0; c < 7; ++c)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        R[c][q] = c == q ? 1.0 : 0.0;
+        V[c][q] = c == q + 3 ? 1.0 : 0.0;
+      }
+    const int stop = min((chunk + 1) * kChunk, a.nsteps);
+#pragma unroll 1
+    for (; step < stop; ++step) {
+      if (step + 1 < end) next = fetch_env(a.env, step + 1, l);
+#pragma unroll 1
       for (int k = 0; k < 3; ++k) {
-        s.x += a.cdt[k] * s.vx;
-        s.y += a.cdt[k] * s.vy;
-        s.z += a.cdt[k] * s.vz;
-        rx[k] = s.x;
-        ry[k] = s.y;
-        rz[k] = s.z;
-        ux[k] = s.vx;
-        uy[k] = s.vy;
-        uz[k] = s.vz;
-        if (k < 2) {
-          double ax, ay, az;
-          group_acceleration(s, p, gmask, env[k], atm, x, parity, ax, ay, az);
-          s.vx += a.ddt[k] * ax;
-          s.vy += a.ddt[k] * ay;
-          s.vz += a.ddt[k] * az;
-        }
-      }
-      // reverse sweep
-      lvx += a.cdt[3] * lx;
-      lvy += a.cdt[3] * ly;
-      lvz += a.cdt[3] * lz;
+        const double cdt = a.cdt[k], ddt = a.ddt[k];
+        drift(s, cdt);
+        Jacobian j{};
+        double acc[3];
+        total_acceleration<true>(s, p, mask, stage[step & 1][k], atm, acc, j);
+        kick(s, ddt, acc);
+        const double xx = ddt * (j.xx + j.d[0][0]), xy = ddt * (j.xy + j.d[0][1]), xz = ddt * (j.xz + j.d[0][2]);
+        const double yx = ddt * (j.xy + j.d[1][0]), yy = ddt * (j.yy + j.d[1][1]), yz = ddt * (j.yz + j.d[1][2]);
+        const double zx = ddt * (j.xz + j.d[2][0]), zy = ddt * (j.yz + j.d[2][1]), zz = ddt * (j.zz + j.d[2][2]);
+        const double vxx = ddt * j.vxx, vxy = ddt * j.vxy, vxz = ddt * j.vxz, vyy = ddt * j.vyy, vyz = ddt * j.vyz,
+                     vzz = ddt * j.vzz;
 #pragma unroll
-      for (int k = 2; k >= 0; --k) {
-        const double wx = a.ddt[k] * lvx, wy = a.ddt[k] * lvy, wz = a.ddt[k] * lvz;
-        double g[7];
-        acceleration_vjp(rx[k], ry[k], rz[k], ux[k], uy[k], uz[k], p, gmask, env[k], atm, wx, wy, wz, g[0], g[1],
-                         g[2], g[3], g[4], g[5], g[6]);
-        group_sum<7>(x, parity, g);
-        lx += g[0];
-        ly += g[1];
-        lz += g[2];
-        lvx += g[3];
-        lvy += g[4];
-        lvz += g[5];
-        lbc += g[6];
-        lvx += a.cdt[k] * lx;
-        lvy += a.cdt[k] * ly;
-        lvz += a.cdt[k] * lz;
+        for (int c = 0; c < 7; ++c) {
+          const double ux = V[c][0], uy = V[c][1], uz = V[c][2];
+          const double rx = R[c][0] += cdt * ux, ry = R[c][1] += cdt * uy, rz = R[c][2] += cdt * uz;
+          V[c][0] += xx * rx + xy * ry + xz * rz + vxx * ux + vxy * uy + vxz * uz;
+          V[c][1] += yx * rx + yy * ry + yz * rz + vxy * ux + vyy * uy + vyz * uz;
+          V[c][2] += zx * rx + zy * ry + zz * rz + vxz * ux + vyz * uy + vzz * uz;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) V[6][q] += ddt * j.b[q];
       }
+      const double cdt = a.cdt[3];
+      drift(s, cdt);
+#pragma unroll
+      for (int c = 0; c < 7; ++c)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) R[c][q] += cdt * V[c][q];
+      if (step + 1 < end) keep_env(stage[(step + 1) & 1], next, l);
+    }
+    if (live) {
+      double *out = a.phi + (size_t)(chunk - a.chunk0) * kPhi * n + i;
+#pragma unroll
+      for (int c = 0; c < 7; ++c)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          out[(size_t)(6 * c + q) * n] = R[c][q];
+          out[(size_t)(6 * c + 3 + q) * n] = V[c][q];
+        }
     }
   }
-  if (w == 0 && live) {
-    // dummies: no gradient flows through a deleted object
-    const double keep = moving ? 1.0 : 0.0;
-    a.g_r0[i] = moving ? lx : (a.g_rT ? a.g_rT[i] : 0.0);
-    a.g_r0[n + i] = moving ? ly : (a.g_rT ? a.g_rT[n + i] : 0.0);
-    a.g_r0[2 * n + i] = moving ? lz : (a.g_rT ? a.g_rT[2 * n + i] : 0.0);
-    a.g_v0[i] = moving ? lvx : (a.g_vT ? a.g_vT[i] : 0.0);
-    a.g_v0[n + i] = moving ? lvy : (a.g_vT ? a.g_vT[n + i] : 0.0);
-    a.g_v0[2 * n + i] = moving ? lvz : (a.g_vT ? a.g_vT[2 * n + i] : 0.0);
-    if (a.g_bc) a.g_bc[i] = keep * lbc;
+}
+
+// lambda = Phi^T lambda over the chunks [chunk0, chunk0 + nchunk), last to first.  The first
+// call (the trajectory's last chunks) starts from the loss gradient, the later ones from what
+// the previous call left in the outputs.
+__global__ __launch_bounds__(kAdjLanes) void k_adjoint_chain(AdjointArgs a) {
+  const size_t n = a.n, i = (size_t)blockIdx.x * kAdjLanes + threadIdx.x;
+  if (i >= n) return;
+  const bool first = (a.chunk0 + a.nchunk) * kChunk >= a.nsteps;
+  const double *sr = first ? a.g_rT : a.g_r0, *sv = first ? a.g_vT : a.g_v0;
+  double g[6];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    g[q] = sr ? sr[q * n + i] : 0.0;
+    g[3 + q] = sv ? sv[q * n + i] : 0.0;
   }
+  double gbc = (!first && a.g_bc) ? a.g_bc[i] : 0.0;
+  // dummies: no gradient flows through a deleted object
+  const bool moving = !a.activity || a.activity[i] >= 0;
+#pragma unroll 2
+  for (int c = a.nchunk - 1; c >= 0 && moving; --c) {
+    const double *m = a.phi + (size_t)c * kPhi * n + i;
+    double v[kPhi];
+#pragma unroll
+    for (int q = 0; q < kPhi; ++q) v[q] = m[(size_t)q * n];
+    double h[7];
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+      h[k] = ((v[6 * k] * g[0] + v[6 * k + 1] * g[1]) + v[6 * k + 2] * g[2]) +
+             ((v[6 * k + 3] * g[3] + v[6 * k + 4] * g[4]) + v[6 * k + 5] * g[5]);
+#pragma unroll
+    for (int q = 0; q < 6; ++q) g[q] = h[q];
+    gbc += h[6];
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    a.g_r0[q * n + i] = g[q];
+    a.g_v0[q * n + i] = g[3 + q];
+  }
+  if (a.g_bc) a.g_bc[i] = gbc;
 }
 
 }  // namespace ladds
@@ -427,7 +563,8 @@ struct ladds_adjoint {
   int every = 64, nck = 0;
   std::string err;
   SubstepEnv<double> *env = nullptr;
-  double *work = nullptr;
+  double *phi = nullptr;  // transition matrices of `group` chunks
+  int group = 1;
   double cdt[4], ddt[3];
   int fail(int code, const std::string &m) {
     err = m;
@@ -477,10 +614,15 @@ int ladds_adjoint_create(const ladds_adjoint_config *cfg, ladds_adjoint **out) {
   if (e == hipSuccess) e = hipMemcpyToSymbol(HIP_SYMBOL(c_atm_adj), &t, sizeof(t));
   if (e == hipSuccess) e = hipMalloc(&p->env, sizeof(SubstepEnv<double>) * env.size());
   if (e == hipSuccess) e = hipMemcpy(p->env, env.data(), sizeof(SubstepEnv<double>) * env.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(&p->work, sizeof(double) * 6 * cfg->n * (size_t)p->every);
+  // Matrices of as many chunks at once as 256 MiB hold, or what one segment's states would take
+  // if that is more; at most 1,024 (a grid dimension holds 65,535 segments)
+  const size_t chunk_bytes = sizeof(double) * kPhi * cfg->n, chunks = ((size_t)cfg->nsteps + kChunk - 1) / kChunk;
+  const size_t budget = std::max<size_t>((size_t)256 << 20, sizeof(double) * 6 * cfg->n * (size_t)p->every);
+  p->group = (int)std::min<size_t>({chunks, std::max<size_t>(1, budget / chunk_bytes), 1024});
+  if (e == hipSuccess) e = hipMalloc(&p->phi, chunk_bytes * (size_t)p->group);
   if (e != hipSuccess) {
     hipFree(p->env);
-    hipFree(p->work);
+    hipFree(p->phi);
     delete p;
     return e == hipErrorOutOfMemory ? LADDS_E_NOMEM : LADDS_E_HIP;
   }
@@ -492,7 +634,7 @@ int ladds_adjoint_destroy(ladds_adjoint *p) {
   if (!p) return LADDS_E_INVALID;
   (void)hipSetDevice(p->cfg.device);
   hipFree(p->env);
-  hipFree(p->work);
+  hipFree(p->phi);
   delete p;
   return LADDS_OK;
 }
@@ -513,7 +655,7 @@ static AdjointArgs make_args(const ladds_adjoint *p) {
   for (int k = 0; k < 4; ++k) a.cdt[k] = p->cdt[k];
   for (int k = 0; k < 3; ++k) a.ddt[k] = p->ddt[k];
   a.env = p->env;
-  a.work = p->work;
+  a.phi = p->phi;
   return a;
 }
 
@@ -533,8 +675,13 @@ int ladds_adjoint_forward(ladds_adjoint *p, const double *r0, const double *v0, 
   a.rT = rT;
   a.vT = vT;
   a.ck = checkpoints;
-  const unsigned blocks = (unsigned)((a.n + kAdjLanes - 1) / kAdjLanes);
-  hipLaunchKernelGGL(k_adjoint_forward, dim3(blocks), dim3(kAdjWaves * kAdjLanes), 0, (hipStream_t)stream, a);
+  const bool grouped = a.n <= kGroupObjects;
+  const size_t per_block = grouped ? kAdjLanes : kAdjWaves * kAdjLanes;
+  const dim3 blocks((unsigned)((a.n + per_block - 1) / per_block)), threads(kAdjWaves * kAdjLanes);
+  if (grouped)
+    hipLaunchKernelGGL(k_adjoint_forward<true>, blocks, threads, 0, (hipStream_t)stream, a);
+  else
+    hipLaunchKernelGGL(k_adjoint_forward<false>, blocks, threads, 0, (hipStream_t)stream, a);
   ADJCHK(p, hipGetLastError());
   return LADDS_OK;
 }
@@ -557,8 +704,17 @@ int ladds_adjoint_backward(ladds_adjoint *p, const double *aom, const double *bc
   a.g_v0 = g_v0;
   a.g_bc = g_bc;
   const unsigned blocks = (unsigned)((a.n + kAdjLanes - 1) / kAdjLanes);
-  hipLaunchKernelGGL(k_adjoint_backward, dim3(blocks), dim3(kAdjWaves * kAdjLanes), 0, (hipStream_t)stream, a);
-  ADJCHK(p, hipGetLastError());
+  const int chunks = (a.nsteps + kChunk - 1) / kChunk;
+  for (int end = chunks; end > 0; end -= p->group) {
+    a.chunk0 = std::max(0, end - p->group);
+    a.nchunk = end - a.chunk0;
+    // chunks that begin in one segment are one thread's
+    const int runs = a.every < kChunk ? a.nchunk : (end - 1) * kChunk / a.every - a.chunk0 * kChunk / a.every + 1;
+    hipLaunchKernelGGL(k_adjoint_segments, dim3(blocks, (unsigned)runs), dim3(kAdjLanes), 0, (hipStream_t)stream, a);
+    ADJCHK(p, hipGetLastError());
+    hipLaunchKernelGGL(k_adjoint_chain, dim3(blocks), dim3(kAdjLanes), 0, (hipStream_t)stream, a);
+    ADJCHK(p, hipGetLastError());
+  }
   return LADDS_OK;
 }
 

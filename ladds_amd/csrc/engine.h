@@ -27,7 +27,7 @@ struct SubstepEnv {
   T moon_k;               // GM_moon / |m|^3
   T sun_acc[3];           // GM_sun s / |s|^3   (indirect term of the direct third-body form)
   T moon_acc[3];          // GM_moon m / |m|^3
-  T pad[2];
+  T c2, s2;               // cos/sin of twice the Earth rotation angle (tesseral terms)
 };
 static_assert(sizeof(SubstepEnv<double>) == 20 * 8, "env layout");
 static_assert(sizeof(SubstepEnv<float>) == 20 * 4, "env layout");

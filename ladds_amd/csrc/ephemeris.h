@@ -92,7 +92,8 @@ __host__ __device__ inline void substep_env(double t, SubstepEnv<double> &e64, S
     e64.sun_acc[k] = e64.sun_k * e64.sun[k];
     e64.moon_acc[k] = e64.moon_k * e64.moon[k];
   }
-  e64.pad[0] = e64.pad[1] = 0.0;
+  e64.c2 = e64.ct * e64.ct - e64.st * e64.st;
+  e64.s2 = 2.0 * e64.ct * e64.st;
   e32.ct = (float)e64.ct;
   e32.st = (float)e64.st;
   for (int k = 0; k < 3; ++k) {
@@ -107,7 +108,8 @@ __host__ __device__ inline void substep_env(double t, SubstepEnv<double> &e64, S
     e32.sun_acc[k] = (float)e64.sun_acc[k];
     e32.moon_acc[k] = (float)e64.moon_acc[k];
   }
-  e32.pad[0] = e32.pad[1] = 0.f;
+  e32.c2 = (float)e64.c2;
+  e32.s2 = (float)e64.s2;
 }
 
 void yoshida_coefficients(double c[4], double d[3]);

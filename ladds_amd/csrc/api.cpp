@@ -357,13 +357,14 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     }
     const double nx = std::min(1.0e6, 2.0 * xmax / cell_x + 3.0);
     g.bx = std::min<uint32_t>(14u, std::max<uint32_t>(2u, ceil_log2((uint64_t)nx)));
-    // a scenario of an ensemble is a population of its own: its planes hold ~64 objects (or
-    // the tuner's choice), folding distant x-slabs into one plane so that the per-plane
-    // set-up of the pair kernel is spread over enough objects
+    // Distant x-slabs are folded into one plane until planes hold ~32 objects, or ~256 of a
+    // scenario of an ensemble (a population of its own) or the tuner's choice, so that a plane's
+    // set-up in the partition and the pair kernel is spread over enough objects (64 scenarios,
+    // sparse pair kernel: 97 us per step with 64 objects, 81 with 256).
     const size_t nscen = ctx->scen_off.size() > 2 ? ctx->scen_off.size() - 1 : 1;
     const size_t per_pop = std::max<size_t>(n / nscen, 1);
-    const size_t ens_plane = ctx->tune_ens_plane > 0 ? (size_t)ctx->tune_ens_plane : 64;
-    if (nscen > 1) g.bx = std::min<uint32_t>(g.bx, std::max<uint32_t>(2u, ceil_log2(per_pop / ens_plane + 1)));
+    const size_t ens_plane = ctx->tune_ens_plane > 0 ? (size_t)ctx->tune_ens_plane : 256;
+    g.bx = std::min<uint32_t>(g.bx, std::max<uint32_t>(2u, ceil_log2(per_pop / (nscen > 1 ? ens_plane : 32) + 1)));
     const uint64_t used = std::min<uint64_t>((uint64_t)nx, 1ull << g.bx);
     uint32_t pb = std::min<uint32_t>(12u, std::max<uint32_t>(4u, ceil_log2(per_pop / used + 1)));
     if (ctx->tune_pb >= 4 && ctx->tune_pb <= 12) pb = (uint32_t)ctx->tune_pb;
@@ -551,6 +552,39 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     ctx->scratch_bytes = arena_bytes;
   }
   tp.arena_cap = (uint32_t)std::min<size_t>(ctx->scratch_bytes / slot_bytes, 0xFFFFFFFFu);
+  // Sparse pair kernel, unless planes are dense (several workgroups each), the tuner asked for
+  // persistent workgroups or the configuration names a workgroup size of the sorting kernel.
+  // Two planes per workgroup where planes are full (1,048,576 objects, split, pair kernel by
+  // events: 33.6 us, one plane 37.3, 512 threads 38.3), 128 threads where they are not (16,384:
+  // 10.4 and 13.6 us).
+  tp.sparse_threads = 0u;
+  if (tiles && !plane_count.empty() && tp.nchunk == 1 && tp.persistent_groups == 0u && !valid_pair_threads(bs)) {
+    // most records of a group of planes and the next one, with room for their drift
+    auto group_max = [&](size_t group) {
+      const size_t P = tp.nplanes;
+      size_t most = 0;
+      for (size_t sc = 0; sc < plane_count.size() / P; ++sc)
+        for (size_t p = 0; p < P; p += group) {
+          size_t k = 0;
+          for (size_t q = 0; q <= group; ++q) k += plane_count[sc * P + (p + q) % P];
+          most = std::max(most, k);
+        }
+      return (most + most / 32 + 32 + 63) / 64 * 64;
+    };
+    auto set = [&](uint32_t threads, uint32_t group, size_t cap) {
+      tp.sparse_threads = threads;
+      tp.sparse_group = group;
+      tp.sparse_cap = (uint32_t)std::min<size_t>(cap, kSparseMost);
+      tp.sparse_list = std::max(64u, tp.sparse_cap / 3);
+    };
+    const size_t cap1 = group_max(1), cap2 = group_max(2);
+    const size_t mean = n / ((size_t)tp.nplanes * tp.nscen);
+    if (mean >= 400 && cap2 <= kSparseMost)
+      set(256, 2, cap2);
+    else if (cap1 <= kSparseMost)
+      set(mean >= 200 ? 256 : 128, 1, cap1);
+    if (tp.sparse_threads && pair_sparse_lds_bytes(tp) > kPairTileLdsBytes) tp.sparse_threads = 0u;
+  }
   ctx->tiles = tp;
   const size_t tps_need = (size_t)tp.ntiles * (tp.nplanes + 1);
   if (tps_need > ctx->tps_alloc) {

@@ -81,6 +81,11 @@ struct TileParams {
   // 1: buckets are two cells wide along z (GridParams::inv_cell_z), and an object scans two
   // buckets of a row, chosen by the half of its bucket it lies in; 0: three buckets.
   uint32_t half_buckets;
+  // > 0: sparse pair kernel (k_pair_sparse) with workgroups of this many threads, each for
+  // sparse_group planes; room for sparse_cap records at a time (at most kSparseMost)
+  // and for sparse_list own records that may have a partner.
+  uint32_t sparse_threads, sparse_group;
+  uint32_t sparse_cap, sparse_list;
   // > 0: the pair kernel runs this many workgroups (as many as the CUs hold at once), each
   // taking plane pairs from its XCD's queue until none is left; 0: one workgroup per plane
   // pair.
@@ -93,6 +98,13 @@ struct TileParams {
 constexpr uint32_t kXcdCount = 8;
 constexpr uint32_t kQueueStride = 32;
 constexpr uint32_t kScanCounterWords = kQueueStride * (1 + kXcdCount);
+
+// Sparse pair kernel: most records it inserts at a time (a node number takes 12 bits), and the
+// folded occupancy map of a plane, one bit per cell: rows along y of 2^kMapZBits cells along z.
+constexpr uint32_t kSparseMost = 4032;
+constexpr uint32_t kMapYBits = 7;
+constexpr uint32_t kMapZBits = 8;
+constexpr uint32_t kMapWords = 1u << (kMapYBits + kMapZBits - 5);
 
 // Sorted record of the plain FP64 form and of the split form: the position the
 // object is binned by, and its index in the object arrays.

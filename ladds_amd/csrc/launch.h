@@ -46,6 +46,8 @@ hipError_t launch_pair_tiles(int form, bool digest, const DeviceObjects &o, cons
                              unsigned long long *log_count, ScanCounters *counters, uint64_t iteration,
                              const StepState *step_state, hipStream_t s);
 uint32_t pair_tiles_header_words(const TileParams &tp);
+// LDS bytes of a workgroup of the sparse pair kernel (TileParams::sparse_threads > 0).
+size_t pair_sparse_lds_bytes(const TileParams &tp);
 // Pair-kernel workgroups of `threads` threads a CU holds by its registers alone (list
 // mode; the persistent instantiation when `persistent`; 0 when the query fails).
 int pair_tiles_groups_per_cu(int form, uint32_t threads, bool persistent = false);

@@ -386,7 +386,7 @@ __device__ __forceinline__ void pair_plane(const PairTileArgs &a, uint32_t *lds,
   if (threadIdx.x == 0) cur_own[-1] = 0;
   __syncthreads();
   const uint32_t total = block_exclusive_scan(seg, 2u * T, wsum);
-  const uint32_t n_own = seg[T];
+  const uint32_t n_own = T ? seg[T] : 0u;  // (a scenario without objects has no tiles)
   if (threadIdx.x == 0) seg[2u * T] = total;
   // chunks this plane uses: ~kChunkRecords own records each, at most tp.nchunk
   const uint32_t cp = min(tp.nchunk, max(1u, (n_own + kChunkRecords - 1u) / kChunkRecords));
@@ -581,6 +581,308 @@ void k_pair_tiles(PairTileArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// sparse pair scan
+// ---------------------------------------------------------------------------
+// One workgroup per GROUP planes and the plane after them, for planes where few objects have
+// another one in the cells around them (1,048,576 objects in low orbits: two in a hundred).
+// Sorting and walking the buckets of every record, the folded grid's aliases included, took 714
+// VALU instructions per record and chains of LDS reads; here the cells around a record are
+// looked up in an occupancy map of one bit per folded cell, and only the records that find
+// one set go on:
+//
+//   insert   every record sets its cell's bit in its plane's map and becomes a node (its
+//            cell, folded beyond any orbit's extent, and the next node) in the chain of its
+//            cell's hash bucket.  A record that finds its bit set shares the cell: its node
+//            says so.
+//   query    every own record reads the 13 cells after its own (z+1; the row y+1; rows y-1,
+//            y, y+1 of the next plane).  If any is set, or it shares its cell, the record and
+//            what it found join a list.
+//   resolve  one thread per listed record walks the chains of the cells it found and lists
+//            the pairs of records it meets; then one thread per pair tests the distance.  In
+//            one cell a record takes those that do not say that they share it (the first one
+//            in) and those of a higher object index.  What passes goes through the exact FP64
+//            predicate.  (Tested where they are met, the few pairs of a wavefront cost one
+//            latency of reading the records after the other: 34 us of 51 at 1,048,576 objects.)
+//
+// Within R, two records' cells differ by at most one along each axis (cells have side >= R),
+// so the record in the earlier cell finds the other's bit, and only that one does: a fold
+// of 2^7 x 2^8 cells cannot turn a cell before into a cell after.  Folding only adds tests.
+// With 2^15 cells per map and ~600 records per plane one own record in four is listed, mostly
+// for an alias, which the node's cell rules out: records are read again (and their place looked
+// up in the segment tables) for true neighbours only.
+//
+// More records than sparse_cap nodes are inserted in turns, each queried by all own records;
+// more listed records than sparse_list are found again in turns of that many.
+constexpr uint32_t kSparseRow = 1u << (kMapZBits - 5);  // words of a map row
+constexpr uint32_t kNodeYBits = 15, kNodeZBits = 15;      // a node's cell, with the plane (0 to GROUP)
+constexpr uint32_t kHeadBits = 10, kHeads = 1u << kHeadBits;  // hash buckets of cells
+constexpr uint32_t kNextBits = 12, kNoNode = (1u << kNextBits) - 1u;  // end of a chain
+constexpr uint32_t kShared = 1u << kNextBits;                         // node: not the first one in its cell
+
+constexpr uint32_t kSparseBatch = 4;                                  // records a thread loads at once
+constexpr uint32_t kPairList = 256;                                   // pairs of records tested together
+
+// LDS words of the sparse kernel: segment tables, maps, bucket heads, nodes, list.
+struct SparseLayout {
+  uint32_t occ, head, cell, next, list, pairs, sums, total;
+};
+__host__ __device__ inline SparseLayout sparse_layout(uint32_t group, uint32_t tiles, uint32_t list, uint32_t cap) {
+  SparseLayout l;
+  l.occ = (2u * (group + 1u) * tiles + 1u + 3u) & ~3u;
+  l.head = l.occ + (group + 1u) * kMapWords;
+  l.cell = l.head + kHeads;
+  l.next = l.cell + cap;  // 16 bits each
+  l.list = l.next + (cap + 1u) / 2u;
+  l.pairs = l.list + list;
+  l.sums = l.pairs + kPairList;
+  l.total = l.sums + kMaxPairThreads / 64 + 1 + 2;
+  return l;
+}
+
+// A record's cell as its node keeps it; the map's row and column are its low bits.
+__device__ __forceinline__ uint32_t node_cell(double y, double z, uint32_t plane, const GridParams &g) {
+  uint32_t low;
+  const uint32_t iy = (uint32_t)cell_axis(y, g.inv_cell, low), iz = (uint32_t)cell_axis(z, g.inv_cell, low);
+  return (plane << (kNodeYBits + kNodeZBits)) | ((iy & ((1u << kNodeYBits) - 1u)) << kNodeZBits) |
+         (iz & ((1u << kNodeZBits) - 1u));
+}
+__device__ __forceinline__ uint32_t cell_plane(uint32_t c) { return c >> (kNodeYBits + kNodeZBits); }
+__device__ __forceinline__ uint32_t cell_y(uint32_t c) { return (c >> kNodeZBits) & ((1u << kNodeYBits) - 1u); }
+__device__ __forceinline__ uint32_t cell_z(uint32_t c) { return c & ((1u << kNodeZBits) - 1u); }
+__device__ __forceinline__ uint32_t cell_hash(uint32_t c) { return (c * 0x9E3779B1u) >> (32 - kHeadBits); }
+
+// Bits z-1, z, z+1 (bit 0: z-1) of row y of a map.
+__device__ __forceinline__ uint32_t row_bits(const uint32_t *map, uint32_t y, uint32_t z) {
+  const uint32_t z0 = (z - 1u) & ((1u << kMapZBits) - 1u), w = z0 >> 5;
+  const uint32_t *r = map + (y & ((1u << kMapYBits) - 1u)) * kSparseRow;
+  return __builtin_amdgcn_alignbit(r[(w + 1u) & (kSparseRow - 1u)], r[w], z0 & 31u) & 7u;
+}
+
+// What a listed record found: bit 0 its own cell, bit 1 the next cell of its row, bits 2-4
+// row y+1, bits 5-13 rows y-1, y, y+1 of the next plane.
+__device__ __forceinline__ uint32_t found_cell(uint32_t c, uint32_t bit) {
+  const uint32_t row = bit < 2u ? 0u : 1u + (bit - 2u) / 3u;  // 0: own; 1: y+1; 2-4: next plane, y-1 to y+1
+  const uint32_t col = bit < 2u ? bit + 1u : (bit - 2u) % 3u;  // 0: z-1
+  const uint32_t y = cell_y(c) + (row < 2u ? row : row - 3u), z = cell_z(c) + col - 1u;
+  return ((cell_plane(c) + (row >= 2u ? 1u : 0u)) << (kNodeYBits + kNodeZBits)) |
+         ((y & ((1u << kNodeYBits) - 1u)) << kNodeZBits) | (z & ((1u << kNodeZBits) - 1u));
+}
+
+template <int FORM, bool DIGEST, int THREADS, int GROUP>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(5)))
+void k_pair_sparse(PairTileArgs a) {
+  extern __shared__ uint32_t lds[];
+  using REC = RecOf<FORM>;
+  const TileParams &tp = a.tp;
+  ScanAcc acc;
+  const uint32_t P = tp.nplanes;
+  uint32_t wid = xcd_local_item(blockIdx.x, gridDim.x) * GROUP;  // first plane of the group
+  if (tp.plane_order) wid = tp.plane_order[wid];                 // (runs of 8 planes)
+  const uint32_t scen = wid / P, plane0 = wid - scen * P;
+  const uint32_t t0 = tp.scen_tile ? tp.scen_tile[scen] : 0u;
+  const uint32_t T = tp.scen_tile ? tp.scen_tile[scen + 1] - t0 : tp.ntiles;
+  const uint32_t cap = tp.sparse_cap, list_cap = tp.sparse_list;
+  const SparseLayout lay = sparse_layout(GROUP, tp.nscen > 1 ? tp.max_scen_tiles : tp.ntiles, list_cap, cap);
+  const uint32_t S = (GROUP + 1u) * T;  // segments: plane by plane, the records of each tile
+  uint32_t *seg = lds, *src = seg + (S + 1u);
+  uint32_t *occ = lds + lay.occ, *head = lds + lay.head, *cell = lds + lay.cell, *list = lds + lay.list;
+  uint16_t *link = reinterpret_cast<uint16_t *>(lds + lay.next);
+  uint32_t *pair = lds + lay.pairs;
+  uint32_t *wsum = lds + lay.sums, *listed = wsum + kMaxPairThreads / 64 + 1, *pairs = listed + 1;
+  const REC *items = static_cast<const REC *>(a.items);
+  for (uint32_t t = threadIdx.x; t < S; t += THREADS) {
+    const uint32_t p = t / T, g = t0 + (t - p * T);
+    const uint32_t *row = a.tps + (size_t)g * (P + 1) + ((plane0 + p) & (P - 1u));
+    const uint32_t o0 = row[0], o1 = row[1];
+    seg[t] = o1 - o0;
+    src[t] = (tp.tile_begin ? tp.tile_begin[g] : g * tp.tile_size) + o0;
+  }
+  auto clear = [&] {
+    uint4 *m = reinterpret_cast<uint4 *>(occ);
+    for (uint32_t k = threadIdx.x; k < (GROUP + 1u) * kMapWords / 4u; k += THREADS) m[k] = make_uint4(0, 0, 0, 0);
+    m = reinterpret_cast<uint4 *>(head);
+    for (uint32_t k = threadIdx.x; k < kHeads / 4u; k += THREADS) m[k] = make_uint4(kNoNode, kNoNode, kNoNode, kNoNode);
+    if (threadIdx.x == 0) *listed = *pairs = 0;
+  };
+  clear();
+  __syncthreads();
+  const uint32_t total = block_exclusive_scan(seg, S, wsum);
+  const uint32_t n_own = T ? seg[GROUP * T] : 0u;  // (a scenario without objects has no tiles)
+  if (n_own == 0u) return;
+  const uint32_t end0 = seg[T], end1 = GROUP > 1 ? seg[2u * T] : total;
+  if (threadIdx.x == 0) seg[S] = total;
+  __syncthreads();
+  // segment of record j
+  auto find = [&](uint32_t j) -> uint32_t {
+    uint32_t lo = 0, hi = S;
+    while (hi - lo > 1u) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (seg[mid] <= j)
+        lo = mid;
+      else
+        hi = mid;
+    }
+    return lo;
+  };
+  auto item_of = [&](uint32_t j) -> uint32_t {
+    const uint32_t t = find(j);
+    return src[t] + (j - seg[t]);
+  };
+  auto plane_of = [&](uint32_t j) -> uint32_t {
+    return (j >= end0 ? 1u : 0u) + ((GROUP > 1 && j >= end1) ? 1u : 0u);
+  };
+#pragma unroll 1
+  for (uint32_t c0 = 0; c0 < total; c0 += cap) {
+    if (c0) {
+      clear();
+      __syncthreads();
+    }
+    // insert the records [c0, c1), a run of them per thread
+    const uint32_t c1 = min(total, c0 + cap);
+    const uint32_t ipt = (c1 - c0 + THREADS - 1u) / THREADS;
+    const uint32_t jb = c0 + threadIdx.x * ipt, je = min(c1, jb + ipt);
+    uint32_t t = jb < je ? find(jb) : 0u;
+#pragma unroll 1
+    for (uint32_t k0 = 0; k0 < ipt; k0 += kSparseBatch) {  // (uniform: every lane takes every batch)
+      decltype(REC::y) y[kSparseBatch], z[kSparseBatch];
+#pragma unroll
+      for (uint32_t k = 0; k < kSparseBatch; ++k) {
+        const uint32_t j = jb + k0 + k;
+        if (j < je) {
+          while (seg[t + 1u] <= j) ++t;
+          const REC *r = items + src[t] + (j - seg[t]);
+          y[k] = r->y;
+          z[k] = r->z;
+        }
+      }
+#pragma unroll
+      for (uint32_t k = 0; k < kSparseBatch; ++k) {
+        const uint32_t j = jb + k0 + k;
+        if (j < je) {
+          const uint32_t p = plane_of(j), c = node_cell((double)y[k], (double)z[k], p, a.g);
+          const uint32_t bit = 1u << (cell_z(c) & 31u);
+          const uint32_t word = p * kMapWords + (cell_y(c) & ((1u << kMapYBits) - 1u)) * kSparseRow +
+                                ((cell_z(c) & ((1u << kMapZBits) - 1u)) >> 5);
+          const uint32_t shared = (atomicOr(&occ[word], bit) & bit) ? kShared : 0u;
+          const uint32_t prev = atomicExch(&head[cell_hash(c)], j - c0);
+          cell[j - c0] = c;
+          link[j - c0] = (uint16_t)(shared | prev);
+        }
+      }
+    }
+    __syncthreads();
+    const bool whole = total <= cap;
+    uint32_t turn = min(n_own, 1u << 18);  // own records queried per turn (a list entry holds 18 bits)
+#pragma unroll 1
+    for (uint32_t b0 = 0; b0 < n_own;) {
+      const uint32_t b1 = min(n_own, b0 + turn);
+#pragma unroll 1
+      for (uint32_t jj = b0; jj < b1; jj += THREADS) {
+        const uint32_t j = jj + threadIdx.x;
+        uint32_t found = 0;
+        if (j < b1) {
+          uint32_t c;
+          if (whole) {
+            c = cell[j];
+            found = (link[j] & kShared) ? 1u : 0u;
+          } else {
+            const REC r = items[item_of(j)];
+            c = node_cell((double)r.y, (double)r.z, plane_of(j), a.g);
+            found = 1u;  // any record of this turn may share the cell
+          }
+          const uint32_t *own = occ + cell_plane(c) * kMapWords, *nxt = own + kMapWords;
+          const uint32_t fy = cell_y(c), fz = cell_z(c);
+          found |= (row_bits(own, fy, fz) & 4u) >> 1;
+          found |= row_bits(own, fy + 1u, fz) << 2;
+          found |= row_bits(nxt, fy - 1u, fz) << 5;
+          found |= row_bits(nxt, fy, fz) << 8;
+          found |= row_bits(nxt, fy + 1u, fz) << 11;
+        }
+        const unsigned long long m = __ballot(found != 0u);
+        if (m) {
+          uint32_t base = 0;
+          const int leader = __ffsll((long long)m) - 1;
+          if ((int)lane_id() == leader) base = atomicAdd(listed, (uint32_t)__popcll(m));
+          base = __shfl(base, leader, 64);
+          const uint32_t pos = base + (uint32_t)__popcll(m & ((1ull << lane_id()) - 1ull));
+          if (found != 0u && pos < list_cap) list[pos] = ((j - b0) << 14) | found;
+        }
+      }
+      __syncthreads();
+      const uint32_t nf = *listed;
+      const bool fits = nf <= list_cap;
+      if (fits) {
+        // resolve: every thread walks the chains of its listed records and puts the pairs of
+        // records it meets in the pair list; whenever that is full, or all walks have ended,
+        // the workgroup reads those records again and tests them
+        uint32_t f = threadIdx.x, found = 0, c = 0, fc = 0, j = 0, bit = 0, q = kNoNode;
+        auto open = [&] {  // listed record f
+          if (f >= nf) return;
+          const uint32_t e = list[f];
+          j = b0 + (e >> 14);
+          found = e & 0x3FFFu;
+          if (whole) {
+            c = cell[j];
+          } else {
+            const REC r = items[item_of(j)];
+            c = node_cell((double)r.y, (double)r.z, plane_of(j), a.g);
+          }
+        };
+        open();
+#pragma unroll 1
+        for (;;) {
+#pragma unroll 1
+          while (f < nf) {
+            if (q != kNoNode) {
+              const uint32_t n = link[q];
+              if (cell[q] == fc) {
+                const uint32_t pos = atomicAdd(pairs, 1u);
+                if (pos >= kPairList) break;  // again after the list is emptied
+                pair[pos] = ((j - b0) << 14) | (q << 2) | (bit == 0u ? 2u : 0u) | ((n & kShared) ? 1u : 0u);
+              }
+              q = n & kNoNode;
+            } else if (found) {
+              bit = (uint32_t)__ffs((int)found) - 1u;
+              found &= found - 1u;
+              fc = found_cell(c, bit);
+              q = head[cell_hash(fc)];
+            } else {
+              f += THREADS;
+              open();
+            }
+          }
+          __syncthreads();
+          const uint32_t met = *pairs, np = min(met, kPairList);
+#pragma unroll 1
+          for (uint32_t k = threadIdx.x; k < np; k += THREADS) {
+            const uint32_t e = pair[k];
+            const REC me = items[item_of(b0 + (e >> 14))], o = items[item_of(c0 + ((e >> 2) & kNoNode))];
+            // in one cell: the first one in is taken by every other, two others by the lower
+            // index (in turns: by the lower index)
+            const bool take = (e & 2u) == 0u || o.idx > me.idx || (whole && (e & 1u) == 0u);
+            if (take && o.idx != me.idx && within<FORM>(me, o, a.sink.fp))
+              handle_candidate<DIGEST>(a.sink, me.idx, o.idx, acc, scen);
+          }
+          if (met <= kPairList) break;  // no walk was stopped
+          __syncthreads();
+          if (threadIdx.x == 0) *pairs = 0;
+          __syncthreads();
+        }
+        b0 = b1;
+      } else {
+        turn = list_cap;  // this turn again, in smaller ones
+      }
+      if (!(fits && b0 >= n_own && whole)) {  // another turn follows
+        __syncthreads();
+        if (threadIdx.x == 0) *listed = *pairs = 0;
+        __syncthreads();
+      }
+    }
+  }
+  flush_counters<DIGEST>(a.sink, acc);
+}
+
+// ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
 hipError_t launch_bin_keys(int form, const DeviceObjects &o, const GridParams &g, uint32_t *keys, hipStream_t s) {
@@ -660,6 +962,19 @@ hipError_t set_pair_lds_limit(int max_lds) {
   return e;
 }
 
+template <int THREADS, int GROUP>
+hipError_t set_sparse_lds_limit(int max_lds) {
+  const void *fs[] = {reinterpret_cast<const void *>(&k_pair_sparse<kFormFp64, false, THREADS, GROUP>),
+                      reinterpret_cast<const void *>(&k_pair_sparse<kFormFp64, true, THREADS, GROUP>),
+                      reinterpret_cast<const void *>(&k_pair_sparse<kFormSplit, false, THREADS, GROUP>),
+                      reinterpret_cast<const void *>(&k_pair_sparse<kFormSplit, true, THREADS, GROUP>)};
+  for (const void *f : fs) {
+    const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 hipError_t configure_tile_kernels() {
   const int max_lds = 160 * 1024;
   hipError_t e = set_pair_lds_limit<128>(max_lds);
@@ -667,6 +982,9 @@ hipError_t configure_tile_kernels() {
   if (e == hipSuccess) e = set_pair_lds_limit<384>(max_lds);
   if (e == hipSuccess) e = set_pair_lds_limit<512>(max_lds);
   if (e == hipSuccess) e = set_pair_lds_limit<1024>(max_lds);
+  if (e == hipSuccess) e = set_sparse_lds_limit<128, 1>(max_lds);
+  if (e == hipSuccess) e = set_sparse_lds_limit<256, 1>(max_lds);
+  if (e == hipSuccess) e = set_sparse_lds_limit<256, 2>(max_lds);
   auto set = [&](const void *f) {
     if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   };
@@ -742,6 +1060,23 @@ void launch_pair_tiles_as(int form, bool digest, const PairTileArgs &a, hipStrea
   if (!tp.arena_fat && !persist) launch_pair_variant<THREADS, false, false>(f64, digest, grid, block, shm, s, a);
 }
 
+size_t pair_sparse_lds_bytes(const TileParams &tp) {
+  const uint32_t tiles = tp.nscen > 1 ? tp.max_scen_tiles : tp.ntiles;
+  return sizeof(uint32_t) * sparse_layout(tp.sparse_group, tiles, tp.sparse_list, tp.sparse_cap).total;
+}
+
+template <int THREADS, int GROUP>
+hipError_t launch_pair_sparse_as(int form, bool digest, const PairTileArgs &a, hipStream_t s) {
+  const size_t shm = pair_sparse_lds_bytes(a.tp);
+  const dim3 grid(a.tp.nplanes / GROUP * a.tp.nscen), block(THREADS);
+  const bool f64 = (form == kFormFp64);
+  if (f64 && !digest) hipLaunchKernelGGL((k_pair_sparse<kFormFp64, false, THREADS, GROUP>), grid, block, shm, s, a);
+  if (f64 && digest) hipLaunchKernelGGL((k_pair_sparse<kFormFp64, true, THREADS, GROUP>), grid, block, shm, s, a);
+  if (!f64 && !digest) hipLaunchKernelGGL((k_pair_sparse<kFormSplit, false, THREADS, GROUP>), grid, block, shm, s, a);
+  if (!f64 && digest) hipLaunchKernelGGL((k_pair_sparse<kFormSplit, true, THREADS, GROUP>), grid, block, shm, s, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_pair_tiles(int form, bool digest, const DeviceObjects &o, const GridParams &g,
                              const TileParams &tp, const FunctorParams &fp, const void *items, const uint32_t *tps,
                              void *scratch, uint32_t *arena_top, LoggedPair *log, uint64_t log_cap,
@@ -756,6 +1091,9 @@ hipError_t launch_pair_tiles(int form, bool digest, const DeviceObjects &o, cons
   a.tps = tps;
   a.scratch = scratch;
   a.arena_top = arena_top;
+  if (tp.sparse_threads == 128) return launch_pair_sparse_as<128, 1>(form, digest, a, s);
+  if (tp.sparse_threads == 256 && tp.sparse_group == 1) return launch_pair_sparse_as<256, 1>(form, digest, a, s);
+  if (tp.sparse_threads == 256 && tp.sparse_group == 2) return launch_pair_sparse_as<256, 2>(form, digest, a, s);
   switch (tp.pair_threads) {
     case 128:
       launch_pair_tiles_as<128>(form, digest, a, s);

@@ -162,6 +162,8 @@ struct ladds_ctx {
   uint32_t *d_plane_order = nullptr;
   size_t plane_order_alloc = 0;
 
+  double crowding = 0.0;  // objects in an object's own cell, from a sample (crowding_of)
+
   // Autotuned plane-tile shape (ladds_autotune); zero / negative values keep the defaults.
   double tune_cell_km = 0.0;
   int tune_pb = -1;
@@ -172,8 +174,8 @@ struct ladds_ctx {
   int tune_wgs = 0;      // pair-kernel workgroups per CU its LDS is sized for (0: automatic)
   int tune_order = 0;    // pair-kernel dispatch: 0 plane order, 1 heaviest runs of planes first
   int tune_ens_plane = 0;  // ensembles: objects per x-plane the planes are sized for (0: 64)
-  int tune_rows = 0;       // bucket row height along y in cells: 2 or 1 (0: 1)
-  int tune_bcells = 0;     // bucket width along z in cells: 2 or 1 (0: 1)
+  int tune_rows = 0;       // bucket row height along y in cells: 2 or 1 (0: by the crowding)
+  int tune_bcells = 0;     // bucket width along z in cells: 2 or 1 (0: by the crowding)
   int tune_persistent = 0; // 1: pair kernel as persistent workgroups with per-XCD queues
   int tune_pair_streams = 0; // pair scans of the overlapped loop on 1 or 2 streams (0: by form)
 
@@ -321,6 +323,54 @@ hipError_t alloc_objects(DeviceObjects &o, size_t cap) {
   return e;
 }
 
+// Mean number of other objects in an object's cell (side `cell`, same scenario), estimated from
+// a sample of at most kCrowdingSample objects spread over the indices; position(i, p) gives
+// the position of object i.  Populations in low orbits have ~1e-3; clusters have their size.
+constexpr size_t kCrowdingSample = 4096;
+// From this many on the sorting kernel with scan_crowded takes over from the sparse one, which
+// lists every pair before it tests any (clustered populations, one screening, split / FP64,
+// sparse against crowded: 131,072 objects with 9.5 conjunctions each 297 / 360 against 248 / 258
+// us, 524,288 with 40 each in FP64 4020 against 859).
+constexpr double kCrowded = 2.0;
+// Four times the buckets per plane: clusters then seldom share one by folding (1,048,576
+// clustered objects, split: 1.70 ms, with twice as many again 2.46).
+constexpr uint32_t kCrowdedBits = 2;
+
+size_t crowding_index(size_t k, size_t m, size_t n) {
+  uint64_t h = (k + 1) * 0x9E3779B97F4A7C15ull;  // a place of its own in the k-th of m equal parts
+  h ^= h >> 32;
+  const size_t lo = k * n / m, hi = (k + 1) * n / m;
+  return lo + (size_t)(h % std::max<size_t>(1, hi - lo));
+}
+
+template <typename F>
+double crowding_of(size_t n, const std::vector<uint64_t> &scen_off, double cell, F &&position) {
+  const size_t m = std::min(n, kCrowdingSample);
+  if (m < 2) return 0.0;
+  std::vector<uint64_t> key(m);
+  size_t scen = 0;
+  for (size_t k = 0; k < m; ++k) {
+    const size_t i = crowding_index(k, m, n);
+    while (scen + 2 < scen_off.size() && i >= scen_off[scen + 1]) ++scen;
+    double p[3];
+    position(k, i, p);
+    uint64_t h = scen;
+    for (int c = 0; c < 3; ++c) {
+      const double u = std::fmin(std::fmax(p[c] / cell, -1.0e9), 1.0e9);
+      h = (h ^ (uint64_t)(int64_t)std::floor(u)) * 0x9E3779B97F4A7C15ull;
+      h ^= h >> 29;
+    }
+    key[k] = h;
+  }
+  std::sort(key.begin(), key.end());
+  double pairs = 0.0;
+  for (size_t k = 0, run = 0; k < m; ++k) {
+    run = (k && key[k] == key[k - 1]) ? run + 1 : 0;
+    pairs += (double)run;
+  }
+  return 2.0 * pairs / (double)m * (double)(n - 1) / (double)(m - 1);
+}
+
 // Grid geometry.  Atomic counting sort: cells of side >= 2R, 2x2x2 search blocks, about
 // one object per bucket.  Plane tiles: cells of side >= R, 3x3x3 neighbourhoods; enough
 // x-planes for the x-extent of the population (no aliasing of x-slabs), about one object
@@ -343,8 +393,9 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   g.inv_cell_x = 1.0 / cell_x;
   // buckets two cells tall (wide): an object then scans two rows of the next plane (two
   // buckets of a row), not three
-  const bool half_rows = tiles && ctx->tune_rows == 2;
-  const bool half_buckets = tiles && ctx->tune_bcells == 2;
+  const bool crowded = ctx->crowding >= kCrowded;
+  const bool half_rows = tiles && (ctx->tune_rows == 2 || (ctx->tune_rows == 0 && crowded));
+  const bool half_buckets = tiles && (ctx->tune_bcells == 2 || (ctx->tune_bcells == 0 && crowded));
   g.inv_cell_y = half_rows ? 0.5 * g.inv_cell : g.inv_cell;
   g.inv_cell_z = half_buckets ? 0.5 * g.inv_cell : g.inv_cell;
   uint32_t bits;
@@ -367,6 +418,7 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     g.bx = std::min<uint32_t>(g.bx, std::max<uint32_t>(2u, ceil_log2(per_pop / (nscen > 1 ? ens_plane : 32) + 1)));
     const uint64_t used = std::min<uint64_t>((uint64_t)nx, 1ull << g.bx);
     uint32_t pb = std::min<uint32_t>(12u, std::max<uint32_t>(4u, ceil_log2(per_pop / used + 1)));
+    if (crowded) pb = std::min<uint32_t>(12u, pb + kCrowdedBits);  // few clusters share a bucket by folding
     if (ctx->tune_pb >= 4 && ctx->tune_pb <= 12) pb = (uint32_t)ctx->tune_pb;
     // rows twice as tall as the buckets are wide fold y with one bit fewer, so that both
     // folds span similar lengths
@@ -448,20 +500,24 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   tp.half_rows = half_rows ? 1u : 0u;
   tp.half_buckets = half_buckets ? 1u : 0u;
   if (tiles && !plane_count.empty() && plane_count.size() == (size_t)tp.nplanes * tp.nscen &&
-      ctx->tune_order == 1) {
+      (ctx->tune_order == 1 || (crowded && !valid_pair_threads(ctx->tune_threads)))) {
     // Dispatch order of the pair kernel's plane pairs (scenario x plane): workgroups start
     // in index order and each XCD takes runs of 8 consecutive plane pairs, so runs of 8
     // planes of one scenario are put in descending order of their work (longest first: the
     // last workgroups on a CU are the short ones).  Work of a plane pair ~ 6 x own records
     // (scan) + next records (gather).  Measured at 1M objects: -6% for FP64 records with
     // 512 threads, +7% for split records with 256 threads, so the tuner decides.
-    const uint32_t P = tp.nplanes, run = 8;
+    // Crowded planes: pairs grow with the square, single planes outweigh many others, and the
+    // walk shares nothing with the neighbouring planes that a run would keep in an XCD's L2.
+    // (1,048,576 clustered objects, split: single planes 1.70 ms, runs of 8 1.89.)
+    const uint32_t P = tp.nplanes, run = crowded ? 1 : 8;
     std::vector<std::pair<uint64_t, uint32_t>> w;
     for (uint32_t sc = 0; sc < tp.nscen; ++sc) {
       const uint32_t *pc = plane_count.data() + (size_t)sc * P;
       for (uint32_t r0 = 0; r0 < P; r0 += run) {
         uint64_t s = 0;
-        for (uint32_t p = r0; p < r0 + run && p < P; ++p) s += 6ull * pc[p] + pc[(p + 1) % P];
+        for (uint32_t p = r0; p < r0 + run && p < P; ++p)
+          s += crowded ? (uint64_t)pc[p] * (pc[p] + 2ull * pc[(p + 1) % P]) : 6ull * pc[p] + pc[(p + 1) % P];
         w.emplace_back(s, sc * P + r0);
       }
     }
@@ -486,6 +542,13 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   tp.pair_threads = valid_pair_threads(bs)
                         ? (uint32_t)bs
                         : (tp.nscen > 1 ? 128u : (ctx->form == kFormFp64 ? 1024u : 256u));
+  if (crowded && !valid_pair_threads(bs)) {
+    // by how full the planes are, 256 / 512 / 1024 threads, us: 64 objects per plane, split
+    // 459 / 473 / 617; 256 per plane, split 1972 / 1696 / 2076, FP64 3003 / 2401 / 2144; 128 per
+    // plane, FP64 904 / 859 / 1133
+    const size_t mean = n / ((size_t)tp.nplanes * tp.nscen);
+    tp.pair_threads = mean < 96 ? 256u : ((ctx->form == kFormFp64 && mean >= 192) ? 1024u : 512u);
+  }
   if (valid_pair_threads(ctx->tune_threads)) tp.pair_threads = (uint32_t)ctx->tune_threads;
   tp.lds_header_words = pair_tiles_header_words(tp);  // depends on the workgroup size
   const size_t rec = (ctx->form == kFormFp64) ? sizeof(RecordF64) : sizeof(RecordF32);
@@ -500,6 +563,9 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   size_t own_max = 0;
   for (uint32_t c : plane_count) own_max = std::max<size_t>(own_max, c);
   tp.nchunk = (uint32_t)std::min<size_t>(16, std::max<size_t>(1, own_max / (4 * (size_t)tp.pair_threads)));
+  // crowded: every chunk sorts the plane again and leaves lanes of the walk idle, so only planes
+  // beyond a CU's share of the objects are divided
+  if (crowded) tp.nchunk = (uint32_t)std::max<size_t>(1, std::min<size_t>(tp.nchunk, own_max * 256 / n));
   if (ctx->cfg.scan_chunks >= 1 && ctx->cfg.scan_chunks <= 32) tp.nchunk = (uint32_t)ctx->cfg.scan_chunks;
   if (ctx->tune_chunks >= 1 && ctx->tune_chunks <= 32) tp.nchunk = (uint32_t)ctx->tune_chunks;
   // LDS of a plane pair: room for the fullest plane pair now, then grown to the whole LDS
@@ -535,30 +601,19 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     const size_t cap = share > hdr + kLdsMargin ? (share - hdr - kLdsMargin) / rec / 64 * 64 : 0;
     tp.cap_items = (uint32_t)std::min(fit, std::max<size_t>(cap, 256));
   }
-  // scratch arena for planes beyond the LDS capacity: every chunk of a plane sorts it.  When
-  // plane pairs exceed the LDS capacity now (dense, clustered populations), each slot also
-  // holds the predicate's fields of its object: their many candidates then read two
-  // contiguous records instead of gathering from the object arrays (2.3x per step on
-  // 8M clustered objects); sparse populations keep the leaner kernel.
-  tp.arena_fat = pair_max > tp.cap_items ? 1u : 0u;
-  const size_t slot_bytes = kArenaSlotBytes + (tp.arena_fat ? kFatRecordBytes : 0);
-  const size_t arena_need = std::max<size_t>(2 * n, 1024) * tp.nchunk;
-  const size_t arena_bytes = arena_need * slot_bytes;
-  if (tiles && arena_bytes > ctx->scratch_bytes) {
-    hipFree(ctx->scratch);
-    ctx->scratch = nullptr;
-    ctx->scratch_bytes = 0;
-    HIPCHK(ctx, hipMalloc(&ctx->scratch, arena_bytes));
-    ctx->scratch_bytes = arena_bytes;
-  }
-  tp.arena_cap = (uint32_t)std::min<size_t>(ctx->scratch_bytes / slot_bytes, 0xFFFFFFFFu);
-  // Sparse pair kernel, unless planes are dense (several workgroups each), the tuner asked for
-  // persistent workgroups or the configuration names a workgroup size of the sorting kernel.
-  // Two planes per workgroup where planes are full (1,048,576 objects, split, pair kernel by
-  // events: 33.6 us, one plane 37.3, 512 threads 38.3), 128 threads where they are not (16,384:
-  // 10.4 and 13.6 us).
+  // Sparse pair kernel, unless cells are crowded, a plane and the next one exceed its LDS, the
+  // configuration or the tuner asked for chunks or persistent workgroups or the configuration names
+  // a workgroup size of the sorting kernel.
+  // Two planes per workgroup where planes are full and enough for every CU (pair kernel by events:
+  // 1,048,576 objects in 1450 planes, split, 33.6 us, one plane 37.3; 524,288 in 720, FP64, 33.2
+  // and 28.9), 128 threads where planes are not full (16,384: 10.4 and 13.6 us with 256). Where
+  // long cells leave few planes, 512 threads and a longer pair list (200,000 objects in 181
+  // planes, split, 62 us; 256 threads 105, the sorting kernel 149; 262,144 in 360: 28, 29 and 54).
   tp.sparse_threads = 0u;
-  if (tiles && !plane_count.empty() && tp.nchunk == 1 && tp.persistent_groups == 0u && !valid_pair_threads(bs)) {
+  const bool chunks_chosen = (ctx->cfg.scan_chunks >= 1 && ctx->cfg.scan_chunks <= 32) ||
+                             (ctx->tune_chunks >= 1 && ctx->tune_chunks <= 32);
+  if (tiles && !plane_count.empty() && !(chunks_chosen && tp.nchunk > 1) && tp.persistent_groups == 0u &&
+      !valid_pair_threads(bs) && !crowded) {
     // most records of a group of planes and the next one, with room for their drift
     auto group_max = [&](size_t group) {
       const size_t P = tp.nplanes;
@@ -579,12 +634,28 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     };
     const size_t cap1 = group_max(1), cap2 = group_max(2);
     const size_t mean = n / ((size_t)tp.nplanes * tp.nscen);
-    if (mean >= 400 && cap2 <= kSparseMost)
+    const size_t used = plane_count.size() - (size_t)std::count(plane_count.begin(), plane_count.end(), 0u);
+    if (mean >= 400 && used >= 1024 && cap2 <= kSparseMost)
       set(256, 2, cap2);
     else if (cap1 <= kSparseMost)
-      set(mean >= 200 ? 256 : 128, 1, cap1);
+      set(mean < 200 ? 128 : (used >= 512 ? 256 : 512), 1, cap1);
     if (tp.sparse_threads && pair_sparse_lds_bytes(tp) > kPairTileLdsBytes) tp.sparse_threads = 0u;
+    // one workgroup does a plane whose records fit (64 scenarios of 1,024 to 65,536 objects:
+    // the fullest planes chunked in the sorting kernel 240 us per step, here 130)
+    if (tp.sparse_threads) tp.nchunk = 1;
   }
+  // scratch arena for planes beyond the LDS capacity: every chunk of a plane sorts it
+  tp.crowded = crowded ? 1u : 0u;
+  const size_t arena_need = std::max<size_t>(2 * n, 1024) * tp.nchunk;
+  const size_t arena_bytes = arena_need * kArenaSlotBytes;
+  if (tiles && arena_bytes > ctx->scratch_bytes) {
+    hipFree(ctx->scratch);
+    ctx->scratch = nullptr;
+    ctx->scratch_bytes = 0;
+    HIPCHK(ctx, hipMalloc(&ctx->scratch, arena_bytes));
+    ctx->scratch_bytes = arena_bytes;
+  }
+  tp.arena_cap = (uint32_t)std::min<size_t>(ctx->scratch_bytes / kArenaSlotBytes, 0xFFFFFFFFu);
   ctx->tiles = tp;
   const size_t tps_need = (size_t)tp.ntiles * (tp.nplanes + 1);
   if (tps_need > ctx->tps_alloc) {
@@ -665,6 +736,33 @@ int settle(ladds_ctx *ctx) {
     const int settle_rc = settle(ctx);     \
     if (settle_rc != LADDS_OK) return settle_rc; \
   } while (0)
+
+// The crowding of the objects on the device (after scenarios or objects changed): the sample's
+// positions are gathered and read back.
+int measure_crowding(ladds_ctx *ctx) {
+  const size_t n = ctx->n, m = std::min(n, kCrowdingSample);
+  ctx->crowding = 0.0;
+  if (m < 2) return LADDS_OK;
+  std::vector<uint32_t> idx(m);
+  std::vector<double> state(6 * m);
+  for (size_t k = 0; k < m; ++k) idx[k] = (uint32_t)crowding_index(k, m, n);
+  char *buf = nullptr;
+  const size_t out = (sizeof(uint32_t) * m + 255) / 256 * 256;
+  HIPCHK(ctx, hipMalloc(reinterpret_cast<void **>(&buf), out + sizeof(double) * 6 * m));
+  double *got = reinterpret_cast<double *>(buf + out);
+  hipError_t e = hipMemcpyAsync(buf, idx.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice, ctx->stream);
+  if (e == hipSuccess)
+    e = launch_gather_state(ctx->d, reinterpret_cast<const uint32_t *>(buf), m, got, ctx->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(state.data(), got, sizeof(double) * 6 * m, hipMemcpyDeviceToHost, ctx->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+  hipFree(buf);
+  if (e != hipSuccess) return ctx->hipfail(e, "crowding sample");
+  ctx->crowding = crowding_of(n, ctx->scen_off, ctx->cfg.cutoff_km, [&](size_t k, size_t, double *p) {
+    for (int c = 0; c < 3; ++c) p[c] = state[6 * k + c];
+  });
+  return LADDS_OK;
+}
 
 int ensure_log(ladds_ctx *ctx, uint64_t cap) {
   if (cap <= ctx->log_cap) return LADDS_OK;
@@ -1387,6 +1485,11 @@ int ladds_set_objects(ladds_ctx *ctx, const ladds_objects *o) {
   rc = reserve_objects(ctx, n, false);
   if (rc != LADDS_OK) return rc;
   ctx->scen_off.clear();  // a new population is a single scenario until ladds_set_scenarios
+  ctx->crowding = crowding_of(n, ctx->scen_off, ctx->cfg.cutoff_km, [&](size_t, size_t i, double *p) {
+    p[0] = o->rx[i];
+    p[1] = o->ry[i];
+    p[2] = o->rz[i];
+  });
   rc = setup_grid(ctx, n, o->rx);
   if (rc != LADDS_OK) return rc;
   ctx->n = n;
@@ -1412,6 +1515,8 @@ int ladds_add_objects(ladds_ctx *ctx, const ladds_objects *o) {
   ctx->n = n;
   ctx->d.n = n;
   ctx->protected_objects = ctx->protected_objects || has_parents(o);
+  rc = measure_crowding(ctx);
+  if (rc != LADDS_OK) return rc;
   std::vector<double> rx(n);
   HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * n, hipMemcpyDeviceToHost));
   return setup_grid(ctx, n, rx.data());
@@ -1432,6 +1537,8 @@ int ladds_set_scenarios(ladds_ctx *ctx, size_t nscenarios, const uint64_t *offse
     ctx->scen_off.clear();
   else
     ctx->scen_off.assign(offsets, offsets + nscenarios + 1);
+  const int rc = measure_crowding(ctx);
+  if (rc != LADDS_OK) return rc;
   std::vector<double> rx(ctx->n);
   HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * ctx->n, hipMemcpyDeviceToHost));
   return setup_grid(ctx, ctx->n, rx.data());
@@ -1705,7 +1812,9 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
   // tile, chunks, workgroups per CU, dispatch order, ensemble objects per plane (0: 64), row
   // height and bucket width in cells, persistent pair kernel, pair-scan streams (0: by form)}
   double cur_cell = base_cell, cur_fx = 1.0;
-  int cur[11] = {-1, (int)ctx->tiles.pair_threads, (int)ctx->tiles.tile_size, (int)ctx->tiles.nchunk, 0, 0, 0, 1, 1, 0, 0};
+  int cur[11] = {-1, (int)ctx->tiles.pair_threads, (int)ctx->tiles.tile_size, (int)ctx->tiles.nchunk, 0,
+                 ctx->tiles.plane_order ? 1 : 0, 0, ctx->tiles.half_rows ? 2 : 1, ctx->tiles.half_buckets ? 2 : 1,
+                 0, 0};
   double default_us = 0.0;
   // the objective: one detection, or (ladds_config.tune_simulate) a burst of simulate steps
   auto measure = [&](double *t) {
@@ -1916,8 +2025,8 @@ int ladds_set_tuning(ladds_ctx *ctx, const ladds_tuning *t) {
   ctx->tune_wgs = t->workgroups_per_cu;
   ctx->tune_order = t->plane_order;
   ctx->tune_ens_plane = t->ensemble_plane_objects;
-  ctx->tune_rows = t->row_cells;
-  ctx->tune_bcells = t->bucket_cells;
+  ctx->tune_rows = std::max(1, t->row_cells);  // 0 in a tuning: 1
+  ctx->tune_bcells = std::max(1, t->bucket_cells);
   ctx->tune_persistent = t->persistent;
   ctx->tune_pair_streams = t->pair_streams;
   if (ctx->n == 0) return LADDS_OK;  // applied at the next ladds_set_objects

@@ -66,11 +66,9 @@ struct TileParams {
   // the plane itself (grid: nchunk workgroups per plane, the unused ones exit).
   uint32_t nchunk;
   uint32_t arena_cap;          // records of the global scratch arena
-  // 1: the arena holds arena_cap slots of kArenaSlotBytes (sorted records) followed by
-  // arena_cap predicate records (kFatRecordBytes each) at the same positions, and the pair
-  // kernel's arena planes read the predicate's fields from them (set when plane pairs
-  // exceeded the LDS capacity at set-up: dense, clustered populations)
-  uint32_t arena_fat;
+  // 1: cells hold several objects within the search radius of each other (clusters): the sorting
+  // kernel walks crowded buckets with whole wavefronts (scan_crowded)
+  uint32_t crowded;
   // The plane pairs (scenario * nplanes + plane) in dispatch order (nscen * nplanes
   // entries), or null for index order.
   const uint32_t *plane_order;

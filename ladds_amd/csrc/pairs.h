@@ -30,8 +30,8 @@ __device__ __forceinline__ double dot3(double a0, double a1, double a2, double b
   return exact_dot3(a0, a1, a2, b0, b1, b2);
 }
 
-// What the predicate reads of one object: object `i` of the object arrays, or a copy of
-// its fields stored beside the sorted records of a dense plane pair (FatRecord).
+// What the predicate reads of one object: object `i` of the object arrays, or its fields held
+// in registers (HeldObject).
 struct SoAObject {
   const DeviceObjects &o;
   uint32_t i;
@@ -47,43 +47,68 @@ struct SoAObject {
   __device__ __forceinline__ double vz() const { return o.vz[i]; }
 };
 
-struct alignas(16) FatRecord {
-  double r[3], v[3];
-  double radius_m;
-  uint64_t parent, id;
-  int32_t activity;
-  uint32_t pad;
+// One object's fields in registers: read from the object arrays (`load`), or through the scalar
+// cache when the index is the same for the whole wavefront (`load_uniform`; the kernels that
+// use it do not write the object arrays).
+struct HeldObject {
+  int act;
+  uint64_t par, ident;
+  double rad, r[3], v[3];
+  __device__ __forceinline__ void load(const DeviceObjects &o, uint32_t i) {
+    act = o.activity[i];
+    rad = o.radius_m[i];
+    par = o.parent[i];
+    ident = o.id[i];
+    r[0] = o.rx[i];
+    r[1] = o.ry[i];
+    r[2] = o.rz[i];
+    v[0] = o.vx[i];
+    v[1] = o.vy[i];
+    v[2] = o.vz[i];
+  }
+  template <typename T>
+  static __device__ __forceinline__ T scalar(const T *p, uint32_t i) {
+    typedef const __attribute__((address_space(4))) T *Constant;
+    return ((Constant)(uintptr_t)p)[i];
+  }
+  __device__ __forceinline__ void load_uniform(const DeviceObjects &o, uint32_t i) {
+    act = scalar(o.activity, i);
+    rad = scalar(o.radius_m, i);
+    par = scalar(o.parent, i);
+    ident = scalar(o.id, i);
+    r[0] = scalar(o.rx, i);
+    r[1] = scalar(o.ry, i);
+    r[2] = scalar(o.rz, i);
+    v[0] = scalar(o.vx, i);
+    v[1] = scalar(o.vy, i);
+    v[2] = scalar(o.vz, i);
+  }
+  __device__ __forceinline__ int activity() const { return act; }
+  __device__ __forceinline__ double radius() const { return rad; }
+  __device__ __forceinline__ uint64_t parent() const { return par; }
+  __device__ __forceinline__ uint64_t id() const { return ident; }
+  __device__ __forceinline__ double rx() const { return r[0]; }
+  __device__ __forceinline__ double ry() const { return r[1]; }
+  __device__ __forceinline__ double rz() const { return r[2]; }
+  __device__ __forceinline__ double vx() const { return v[0]; }
+  __device__ __forceinline__ double vy() const { return v[1]; }
+  __device__ __forceinline__ double vz() const { return v[2]; }
 };
 
-__device__ __forceinline__ FatRecord fat_record_of(const DeviceObjects &o, uint32_t i) {
-  FatRecord f;
-  f.r[0] = o.rx[i];
-  f.r[1] = o.ry[i];
-  f.r[2] = o.rz[i];
-  f.v[0] = o.vx[i];
-  f.v[1] = o.vy[i];
-  f.v[2] = o.vz[i];
-  f.radius_m = o.radius_m[i];
-  f.parent = o.parent[i];
-  f.id = o.id[i];
-  f.activity = o.activity[i];
-  f.pad = 0;
-  return f;
+// The one of two held objects that comes first (or second) in index order.
+__device__ __forceinline__ HeldObject chosen(bool first, const HeldObject &a, const HeldObject &b) {
+  HeldObject h;
+  h.act = first ? a.act : b.act;
+  h.par = first ? a.par : b.par;
+  h.ident = first ? a.ident : b.ident;
+  h.rad = first ? a.rad : b.rad;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    h.r[k] = first ? a.r[k] : b.r[k];
+    h.v[k] = first ? a.v[k] : b.v[k];
+  }
+  return h;
 }
-
-struct FatObject {
-  const FatRecord &f;
-  __device__ __forceinline__ int activity() const { return f.activity; }
-  __device__ __forceinline__ double radius() const { return f.radius_m; }
-  __device__ __forceinline__ uint64_t parent() const { return f.parent; }
-  __device__ __forceinline__ uint64_t id() const { return f.id; }
-  __device__ __forceinline__ double rx() const { return f.r[0]; }
-  __device__ __forceinline__ double ry() const { return f.r[1]; }
-  __device__ __forceinline__ double rz() const { return f.r[2]; }
-  __device__ __forceinline__ double vx() const { return f.v[0]; }
-  __device__ __forceinline__ double vy() const { return f.v[1]; }
-  __device__ __forceinline__ double vz() const { return f.v[2]; }
-};
 
 // Returns 0 (no report), 1 (collision) or 2 (evaded); objects `a` (index i) and `b`
 // (index j), i < j, evaluated as AoSFunctor(i, j).
@@ -242,15 +267,13 @@ __device__ __forceinline__ void handle_candidate(const PairSink &a, uint32_t oi,
   sink_result<DIGEST>(a, kind, r, acc, scenario);
 }
 
-// The same predicate with both objects' fields read from their FatRecords fi (object oi)
-// and fj (object oj).
+// The same predicate with both objects held in registers.
 template <bool DIGEST>
-__device__ __forceinline__ void handle_candidate(const PairSink &a, const FatRecord &fi, const FatRecord &fj,
+__device__ __forceinline__ void handle_candidate(const PairSink &a, const HeldObject &hi, const HeldObject &hj,
                                                  uint32_t oi, uint32_t oj, ScanAcc &acc, uint32_t scenario) {
   const bool lo = oi < oj;
   PairRecord r;
-  const int kind = collision_functor(FatObject{lo ? fi : fj}, FatObject{lo ? fj : fi}, lo ? oi : oj, lo ? oj : oi,
-                                     a.fp, r);
+  const int kind = collision_functor(chosen(lo, hi, hj), chosen(lo, hj, hi), lo ? oi : oj, lo ? oj : oi, a.fp, r);
   sink_result<DIGEST>(a, kind, r, acc, scenario);
 }
 

@@ -232,13 +232,11 @@ __device__ __forceinline__ bool within(const RecOf<FORM> &a, const RecOf<FORM> &
 // next), so bucket b spans [cur[b-1], cur[b]).  The rows are
 // walked by one loop so that the candidate path (the exact predicate and the wavefront
 // compaction) exists once in the code.
-// `fat` (or null): the predicate records at the sorted positions, for plane pairs sorted in
-// the global arena.
 template <int FORM, bool DIGEST, bool CHUNKED>
 __device__ __forceinline__ void scan_plane(const PairTileArgs &a, const RecOf<FORM> *sorted,
                                            const uint32_t *cur_own, const uint32_t *cur_halo, uint32_t n_own,
                                            uint32_t threads, uint32_t scen, uint32_t chunk, uint32_t nchunk,
-                                           const FatRecord *fat, ScanAcc &acc) {
+                                           ScanAcc &acc) {
   const GridParams &g = a.g;
   const uint32_t my = (1u << g.by) - 1u, mz = (1u << g.bz) - 1u;
   const uint32_t sy = g.bz;
@@ -324,11 +322,7 @@ __device__ __forceinline__ void scan_plane(const PairTileArgs &a, const RecOf<FO
 #pragma unroll 1
             for (int u = 0; u < 2; ++u) {
               if (!(u ? c1 : c0)) continue;
-              const uint32_t oj = u ? o1.idx : o0.idx;
-              if (fat)
-                handle_candidate<DIGEST>(a.sink, fat[s], fat[q + (uint32_t)u], me.idx, oj, acc, scen);
-              else
-                handle_candidate<DIGEST>(a.sink, me.idx, oj, acc, scen);
+              handle_candidate<DIGEST>(a.sink, me.idx, u ? o1.idx : o0.idx, acc, scen);
             }
           }
         }
@@ -339,12 +333,122 @@ __device__ __forceinline__ void scan_plane(const PairTileArgs &a, const RecOf<FO
   }
 }
 
+// scan_plane for crowded planes: clusters put tens to thousands of records into one cell, all
+// within R of each other, and nearly every record met is a candidate.  A wavefront takes 64
+// consecutive sorted records, and where their runs in a row nearly coincide (one bucket, or a few
+// neighbours) it walks the union of the runs together: the other record, and its predicate
+// fields read through the scalar cache one ahead, are the same for all lanes, and the own
+// fields stay in registers.  Walked lane by lane, every lane met another record and gathered
+// its fields from eleven arrays (or an 80-byte copy), which bounded the scan.  Runs that do not
+// coincide are walked lane by lane as in scan_plane.  Now bounded by the predicate's FP64
+// instructions in half-filled wavefronts and the fullest planes.  One screening of clustered
+// objects, lane by lane -> here: 1,048,576 with 42 million conjunctions, split 6.38 -> 1.70 ms,
+// FP64 11.2 -> 2.14; 131,072 with 0.62 million, split 0.28 -> 0.25, FP64 0.48 -> 0.26.
+template <int FORM, bool DIGEST>
+__device__ __forceinline__ void scan_crowded(const PairTileArgs &a, const RecOf<FORM> *sorted,
+                                             const uint32_t *cur_own, const uint32_t *cur_halo, uint32_t n_own,
+                                             uint32_t threads, uint32_t scen, uint32_t chunk, uint32_t nchunk,
+                                             ScanAcc &acc) {
+  const GridParams &g = a.g;
+  const uint32_t my = (1u << g.by) - 1u, mz = (1u << g.bz) - 1u;
+  const uint32_t sy = g.bz, lane = lane_id();
+  const bool half = a.tp.half_rows != 0u;
+#pragma unroll 1
+  for (uint32_t s0 = threadIdx.x & ~63u; s0 < n_own; s0 += threads) {
+    const uint32_t s = s0 + lane;
+    const RecOf<FORM> me = sorted[min(s, n_own - 1u)];
+    double x, y, z;
+    binning_point_of(me, x, y, z);
+    uint32_t ly, lz;
+    const uint32_t lb = yz_bucket(y, z, g, ly, lz);
+    const uint32_t fy = (lb >> sy) & my, fz = lb & mz;
+    // the chunks of a plane share its buckets
+    const bool on = s < n_own && (nchunk == 1u || lb % nchunk == chunk);
+    if (!__ballot(on)) continue;
+    HeldObject mine;
+    mine.load(a.sink.o, me.idx);
+    uint32_t zlo, zhi;
+    bool wraps;
+    if (a.tp.half_buckets == 0u) {
+      zlo = fz ? fz - 1u : 0u;
+      zhi = fz < mz ? fz + 1u : mz;
+      wraps = (fz == 0u) || (fz == mz);
+    } else {
+      const bool wl = fz == 0u && lz != 0u, wh = fz == mz && lz == 0u;
+      zlo = wl ? 0u : fz - lz;
+      zhi = wh ? mz : fz + 1u - lz;
+      wraps = wl || wh;
+    }
+    const uint32_t zw = fz ? 0u : mz;
+#pragma unroll 1
+    for (uint32_t kind = 0; kind < (half ? 4u : 6u); ++kind) {
+      const bool next_plane = (kind & 1u) != 0u;
+      uint32_t d;
+      bool skip = !on;
+      if (!half) {
+        skip = skip || (kind == 0u && fy != 0u);
+        d = (kind >> 1) - 1u;
+      } else if (next_plane) {
+        d = (kind >> 1) - ly;
+      } else {
+        skip = skip || (kind == 0u && ly != 0u && fy != 0u);
+        d = kind == 2u ? 0u : (ly ? ~0u : 1u);
+      }
+      const uint32_t *cur = next_plane ? cur_halo : cur_own;
+      const uint32_t row = ((fy + d) & my) << sy;
+      const uint32_t from = next_plane ? 0u : s + 1u;
+#pragma unroll 1
+      for (int part = 0; part < 2; ++part) {
+        const uint32_t b0 = row | (part ? zw : zlo), b1 = row | (part ? zw : zhi);
+        const uint32_t lo = cur[(int32_t)b0 - 1], end = cur[b1];
+        uint32_t q = max(lo, from);
+        const bool any = !skip && (part == 0 || wraps) && q < end;
+        const unsigned long long m = __ballot(any);
+        if (!m) continue;
+        const int l0 = __ffsll((long long)m) - 1, l1 = 63 - __clzll((long long)m);
+        const uint32_t first = __builtin_amdgcn_readlane(q, l0), last = __builtin_amdgcn_readlane(end, l1);
+        const uint32_t length = __builtin_amdgcn_readlane(end - lo, l0);
+        const bool apart = __ballot(any && (q < first || end > last)) != 0ull || last - first > 2u * length ||
+                           __popcll(m) < 8;
+        if (!apart) {
+          // the next record and its fields are on their way while this one is tested
+          RecOf<FORM> o = sorted[first];
+          uint32_t oj = __builtin_amdgcn_readfirstlane(o.idx);
+          HeldObject other;
+          other.load_uniform(a.sink.o, oj);
+#pragma unroll 1
+          for (uint32_t u = first; u < last; ++u) {
+            const RecOf<FORM> p = sorted[min(u + 1u, last - 1u)];
+            const uint32_t nj = __builtin_amdgcn_readfirstlane(p.idx);
+            HeldObject following;
+            following.load_uniform(a.sink.o, nj);
+            const bool c = any && u >= q && u < end && within<FORM>(me, o, a.sink.fp);
+            if (c) handle_candidate<DIGEST>(a.sink, mine, other, me.idx, oj, acc, scen);
+            o = p;
+            oj = nj;
+            other = following;
+          }
+        } else if (any) {
+#pragma unroll 1
+          for (; q < end; ++q) {
+            const RecOf<FORM> o = sorted[q];
+            if (within<FORM>(me, o, a.sink.fp)) {
+              HeldObject other;
+              other.load(a.sink.o, o.idx);
+              handle_candidate<DIGEST>(a.sink, mine, other, me.idx, o.idx, acc, scen);
+            }
+          }
+        }
+      }
+    }
+  }
+}
+
 // One work item of the pair scan: plane pair `wid` = (scenario, plane, chunk), sorted in
 // LDS up to tp.cap_items records, beyond that in the global scratch arena.
-// FAT: plane pairs sorted in the arena carry the predicate's fields beside their records
-// (instantiated only for launches whose shape left plane pairs beyond the LDS, so that the
-// common all-in-LDS case keeps the smaller register footprint).
-template <int FORM, bool DIGEST, int THREADS, bool FAT>
+// CROWDED: scan_crowded (a separate instantiation: the common case keeps the smaller register
+// footprint).
+template <int FORM, bool DIGEST, int THREADS, bool CROWDED>
 __device__ __forceinline__ void pair_plane(const PairTileArgs &a, uint32_t *lds, uint32_t wid, ScanAcc &acc) {
   constexpr int kPairRegItems = kPairRegCapacity / THREADS < 8 ? kPairRegCapacity / THREADS : 8;
   using REC = RecOf<FORM>;
@@ -401,11 +505,6 @@ __device__ __forceinline__ void pair_plane(const PairTileArgs &a, uint32_t *lds,
     __syncthreads();
     if (!in_lds && !misc[1]) return;  // no room: the plane is reported, never written out of bounds
     REC *sorted = in_lds ? lds_items : static_cast<REC *>(a.scratch) + misc[0];
-    // dense plane pairs sorted in the arena: the predicate's fields beside each record
-    FatRecord *fat = (FAT && !in_lds)
-                         ? reinterpret_cast<FatRecord *>(static_cast<char *>(a.scratch) +
-                                                         (size_t)tp.arena_cap * kArenaSlotBytes) + misc[0]
-                         : nullptr;
     // own records at [0, n_own), the next plane's at [n_own, total)
     // Each thread reads a block of consecutive records: one binary search for the
     // block's first record, then a forward walk over the segment boundaries.
@@ -490,25 +589,22 @@ __device__ __forceinline__ void pair_plane(const PairTileArgs &a, uint32_t *lds,
         if (pass == 0) block_exclusive_scan(cur_own, 2u * L + 1u, wsum);
       }
     }
-    // cur[b] now holds the end of bucket b.  Arena plane pairs: the predicate's fields of
-    // every sorted record, written in sorted order (the records are visible to the whole
-    // workgroup after the barrier above)
-    if (fat) {
-      for (uint32_t p = threadIdx.x; p < total; p += THREADS) fat[p] = fat_record_of(a.sink.o, sorted[p].idx);
-      __syncthreads();
-    }
-    if (cp > 1u) {
+    // cur[b] now holds the end of bucket b
+    if constexpr (CROWDED) {
       if (in_lds)
-        scan_plane<FORM, DIGEST, true>(a, lds_items, cur_own, cur_next, n_own, THREADS, scen, chunk, cp, nullptr,
-                                       acc);
+        scan_crowded<FORM, DIGEST>(a, lds_items, cur_own, cur_next, n_own, THREADS, scen, chunk, cp, acc);
       else
-        scan_plane<FORM, DIGEST, true>(a, sorted, cur_own, cur_next, n_own, THREADS, scen, chunk, cp, fat, acc);
+        scan_crowded<FORM, DIGEST>(a, sorted, cur_own, cur_next, n_own, THREADS, scen, chunk, cp, acc);
+    } else if (cp > 1u) {
+      if (in_lds)
+        scan_plane<FORM, DIGEST, true>(a, lds_items, cur_own, cur_next, n_own, THREADS, scen, chunk, cp, acc);
+      else
+        scan_plane<FORM, DIGEST, true>(a, sorted, cur_own, cur_next, n_own, THREADS, scen, chunk, cp, acc);
     } else {
       if (in_lds)
-        scan_plane<FORM, DIGEST, false>(a, lds_items, cur_own, cur_next, n_own, THREADS, scen, 0u, 1u, nullptr,
-                                        acc);
+        scan_plane<FORM, DIGEST, false>(a, lds_items, cur_own, cur_next, n_own, THREADS, scen, 0u, 1u, acc);
       else
-        scan_plane<FORM, DIGEST, false>(a, sorted, cur_own, cur_next, n_own, THREADS, scen, 0u, 1u, fat, acc);
+        scan_plane<FORM, DIGEST, false>(a, sorted, cur_own, cur_next, n_own, THREADS, scen, 0u, 1u, acc);
     }
   }
 }
@@ -528,11 +624,11 @@ __device__ __forceinline__ uint32_t xcd_local_item(uint32_t b, uint32_t g) {
 
 // Occupancy target of the pair kernel: 5 waves per SIMD lets the register allocator keep
 // the split form at 77 VGPRs (list mode), 6 waves per SIMD, instead of 103 (4 waves) with
-// no spills; the FP64 form spills under it below 512 threads and keeps the default there.
-template <int FORM, int THREADS>
-constexpr int kPairWavesPerEu = (FORM == kFormSplit || THREADS >= 512) ? 5 : 1;
+// no spills; the FP64 form spills under it below 512 threads, and scan_crowded with its held
+// objects at any size, and they keep the default.
+template <int FORM, int THREADS, bool CROWDED>
+constexpr int kPairWavesPerEu = (!CROWDED && (FORM == kFormSplit || THREADS >= 512)) ? 5 : 1;
 
-static_assert(sizeof(FatRecord) == kFatRecordBytes, "predicate record size");
 static_assert(sizeof(RecordF64) <= kArenaSlotBytes && sizeof(RecordF32) <= kArenaSlotBytes, "arena slot");
 
 // PERSIST false: one workgroup per plane pair (grid nplanes * nscen * nchunk).
@@ -545,8 +641,8 @@ static_assert(sizeof(RecordF64) <= kArenaSlotBytes && sizeof(RecordF32) <= kAren
 // workgroup reads the same run, so all leave the loop together.  A separate instantiation:
 // the loop around the scan costs registers (96 VGPRs against 77) that the one-item kernel
 // keeps free.
-template <int FORM, bool DIGEST, int THREADS, bool FAT, bool PERSIST>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(kPairWavesPerEu<FORM, THREADS>)))
+template <int FORM, bool DIGEST, int THREADS, bool CROWDED, bool PERSIST>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(kPairWavesPerEu<FORM, THREADS, CROWDED>)))
 void k_pair_tiles(PairTileArgs a) {
   extern __shared__ uint32_t lds[];
   ScanAcc acc;
@@ -554,7 +650,7 @@ void k_pair_tiles(PairTileArgs a) {
   if constexpr (!PERSIST) {
     uint32_t item = xcd_local_item(blockIdx.x, gridDim.x);
     if (a.tp.plane_order) item = a.tp.plane_order[item / nchunk] * nchunk + item % nchunk;
-    pair_plane<FORM, DIGEST, THREADS, FAT>(a, lds, item, acc);
+    pair_plane<FORM, DIGEST, THREADS, CROWDED>(a, lds, item, acc);
   } else {
     // the LDS header's last word, which pair_plane leaves alone (a static __shared__ word
     // would push the kernel past the dynamic LDS limit it is configured with)
@@ -572,7 +668,7 @@ void k_pair_tiles(PairTileArgs a) {
       for (uint32_t i = 0; i < kXcdRun && first + i < total; ++i) {
         uint32_t item = first + i;
         if (a.tp.plane_order) item = a.tp.plane_order[item / nchunk] * nchunk + item % nchunk;
-        pair_plane<FORM, DIGEST, THREADS, FAT>(a, lds, item, acc);
+        pair_plane<FORM, DIGEST, THREADS, CROWDED>(a, lds, item, acc);
         __syncthreads();  // the next item's set-up rewrites the LDS this one read
       }
     }
@@ -620,13 +716,15 @@ constexpr uint32_t kNextBits = 12, kNoNode = (1u << kNextBits) - 1u;  // end of 
 constexpr uint32_t kShared = 1u << kNextBits;                         // node: not the first one in its cell
 
 constexpr uint32_t kSparseBatch = 4;                                  // records a thread loads at once
-constexpr uint32_t kPairList = 256;                                   // pairs of records tested together
+// pairs of records tested together
+__host__ __device__ constexpr uint32_t pair_list_of(uint32_t threads) { return threads > 256u ? 1024u : 256u; }
 
 // LDS words of the sparse kernel: segment tables, maps, bucket heads, nodes, list.
 struct SparseLayout {
   uint32_t occ, head, cell, next, list, pairs, sums, total;
 };
-__host__ __device__ inline SparseLayout sparse_layout(uint32_t group, uint32_t tiles, uint32_t list, uint32_t cap) {
+__host__ __device__ inline SparseLayout sparse_layout(uint32_t threads, uint32_t group, uint32_t tiles, uint32_t list,
+                                                       uint32_t cap) {
   SparseLayout l;
   l.occ = (2u * (group + 1u) * tiles + 1u + 3u) & ~3u;
   l.head = l.occ + (group + 1u) * kMapWords;
@@ -634,7 +732,7 @@ __host__ __device__ inline SparseLayout sparse_layout(uint32_t group, uint32_t t
   l.next = l.cell + cap;  // 16 bits each
   l.list = l.next + (cap + 1u) / 2u;
   l.pairs = l.list + list;
-  l.sums = l.pairs + kPairList;
+  l.sums = l.pairs + pair_list_of(threads);
   l.total = l.sums + kMaxPairThreads / 64 + 1 + 2;
   return l;
 }
@@ -673,6 +771,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(5)))
 void k_pair_sparse(PairTileArgs a) {
   extern __shared__ uint32_t lds[];
   using REC = RecOf<FORM>;
+  constexpr uint32_t kPairList = pair_list_of(THREADS);
   const TileParams &tp = a.tp;
   ScanAcc acc;
   const uint32_t P = tp.nplanes;
@@ -682,7 +781,7 @@ void k_pair_sparse(PairTileArgs a) {
   const uint32_t t0 = tp.scen_tile ? tp.scen_tile[scen] : 0u;
   const uint32_t T = tp.scen_tile ? tp.scen_tile[scen + 1] - t0 : tp.ntiles;
   const uint32_t cap = tp.sparse_cap, list_cap = tp.sparse_list;
-  const SparseLayout lay = sparse_layout(GROUP, tp.nscen > 1 ? tp.max_scen_tiles : tp.ntiles, list_cap, cap);
+  const SparseLayout lay = sparse_layout(THREADS, GROUP, tp.nscen > 1 ? tp.max_scen_tiles : tp.ntiles, list_cap, cap);
   const uint32_t S = (GROUP + 1u) * T;  // segments: plane by plane, the records of each tile
   uint32_t *seg = lds, *src = seg + (S + 1u);
   uint32_t *occ = lds + lay.occ, *head = lds + lay.head, *cell = lds + lay.cell, *list = lds + lay.list;
@@ -940,12 +1039,12 @@ hipError_t launch_tile_partition(int form, const DeviceObjects &o, const uint32_
 }
 
 // The four (form, output) instantiations of one workgroup size, arena layout and mode.
-template <int THREADS, bool FAT, bool PERSIST>
+template <int THREADS, bool CROWDED, bool PERSIST>
 hipError_t set_pair_lds_limit_of(int max_lds) {
-  const void *fs[] = {reinterpret_cast<const void *>(&k_pair_tiles<kFormFp64, false, THREADS, FAT, PERSIST>),
-                      reinterpret_cast<const void *>(&k_pair_tiles<kFormFp64, true, THREADS, FAT, PERSIST>),
-                      reinterpret_cast<const void *>(&k_pair_tiles<kFormSplit, false, THREADS, FAT, PERSIST>),
-                      reinterpret_cast<const void *>(&k_pair_tiles<kFormSplit, true, THREADS, FAT, PERSIST>)};
+  const void *fs[] = {reinterpret_cast<const void *>(&k_pair_tiles<kFormFp64, false, THREADS, CROWDED, PERSIST>),
+                      reinterpret_cast<const void *>(&k_pair_tiles<kFormFp64, true, THREADS, CROWDED, PERSIST>),
+                      reinterpret_cast<const void *>(&k_pair_tiles<kFormSplit, false, THREADS, CROWDED, PERSIST>),
+                      reinterpret_cast<const void *>(&k_pair_tiles<kFormSplit, true, THREADS, CROWDED, PERSIST>)};
   for (const void *f : fs) {
     const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
     if (e != hipSuccess) return e;
@@ -985,6 +1084,7 @@ hipError_t configure_tile_kernels() {
   if (e == hipSuccess) e = set_sparse_lds_limit<128, 1>(max_lds);
   if (e == hipSuccess) e = set_sparse_lds_limit<256, 1>(max_lds);
   if (e == hipSuccess) e = set_sparse_lds_limit<256, 2>(max_lds);
+  if (e == hipSuccess) e = set_sparse_lds_limit<512, 1>(max_lds);
   auto set = [&](const void *f) {
     if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   };
@@ -1038,13 +1138,13 @@ uint32_t pair_tiles_header_words(const TileParams &tp) {
   return (w + 7u) & ~7u;  // 32-byte alignment of the record array
 }
 
-template <int THREADS, bool FAT, bool PERSIST>
+template <int THREADS, bool CROWDED, bool PERSIST>
 void launch_pair_variant(bool f64, bool digest, dim3 grid, dim3 block, size_t shm, hipStream_t s,
                          const PairTileArgs &a) {
-  if (f64 && !digest) hipLaunchKernelGGL((k_pair_tiles<kFormFp64, false, THREADS, FAT, PERSIST>), grid, block, shm, s, a);
-  if (f64 && digest) hipLaunchKernelGGL((k_pair_tiles<kFormFp64, true, THREADS, FAT, PERSIST>), grid, block, shm, s, a);
-  if (!f64 && !digest) hipLaunchKernelGGL((k_pair_tiles<kFormSplit, false, THREADS, FAT, PERSIST>), grid, block, shm, s, a);
-  if (!f64 && digest) hipLaunchKernelGGL((k_pair_tiles<kFormSplit, true, THREADS, FAT, PERSIST>), grid, block, shm, s, a);
+  if (f64 && !digest) hipLaunchKernelGGL((k_pair_tiles<kFormFp64, false, THREADS, CROWDED, PERSIST>), grid, block, shm, s, a);
+  if (f64 && digest) hipLaunchKernelGGL((k_pair_tiles<kFormFp64, true, THREADS, CROWDED, PERSIST>), grid, block, shm, s, a);
+  if (!f64 && !digest) hipLaunchKernelGGL((k_pair_tiles<kFormSplit, false, THREADS, CROWDED, PERSIST>), grid, block, shm, s, a);
+  if (!f64 && digest) hipLaunchKernelGGL((k_pair_tiles<kFormSplit, true, THREADS, CROWDED, PERSIST>), grid, block, shm, s, a);
 }
 
 template <int THREADS>
@@ -1054,15 +1154,15 @@ void launch_pair_tiles_as(int form, bool digest, const PairTileArgs &a, hipStrea
   const size_t shm = sizeof(uint32_t) * tp.lds_header_words + rec * tp.cap_items;
   const dim3 grid(tp.persistent_groups ? tp.persistent_groups : tp.nplanes * tp.nscen * tp.nchunk), block(THREADS);
   const bool f64 = (form == kFormFp64), persist = tp.persistent_groups != 0u;
-  if (tp.arena_fat && persist) launch_pair_variant<THREADS, true, true>(f64, digest, grid, block, shm, s, a);
-  if (tp.arena_fat && !persist) launch_pair_variant<THREADS, true, false>(f64, digest, grid, block, shm, s, a);
-  if (!tp.arena_fat && persist) launch_pair_variant<THREADS, false, true>(f64, digest, grid, block, shm, s, a);
-  if (!tp.arena_fat && !persist) launch_pair_variant<THREADS, false, false>(f64, digest, grid, block, shm, s, a);
+  if (tp.crowded && persist) launch_pair_variant<THREADS, true, true>(f64, digest, grid, block, shm, s, a);
+  if (tp.crowded && !persist) launch_pair_variant<THREADS, true, false>(f64, digest, grid, block, shm, s, a);
+  if (!tp.crowded && persist) launch_pair_variant<THREADS, false, true>(f64, digest, grid, block, shm, s, a);
+  if (!tp.crowded && !persist) launch_pair_variant<THREADS, false, false>(f64, digest, grid, block, shm, s, a);
 }
 
 size_t pair_sparse_lds_bytes(const TileParams &tp) {
   const uint32_t tiles = tp.nscen > 1 ? tp.max_scen_tiles : tp.ntiles;
-  return sizeof(uint32_t) * sparse_layout(tp.sparse_group, tiles, tp.sparse_list, tp.sparse_cap).total;
+  return sizeof(uint32_t) * sparse_layout(tp.sparse_threads, tp.sparse_group, tiles, tp.sparse_list, tp.sparse_cap).total;
 }
 
 template <int THREADS, int GROUP>
@@ -1094,6 +1194,7 @@ hipError_t launch_pair_tiles(int form, bool digest, const DeviceObjects &o, cons
   if (tp.sparse_threads == 128) return launch_pair_sparse_as<128, 1>(form, digest, a, s);
   if (tp.sparse_threads == 256 && tp.sparse_group == 1) return launch_pair_sparse_as<256, 1>(form, digest, a, s);
   if (tp.sparse_threads == 256 && tp.sparse_group == 2) return launch_pair_sparse_as<256, 2>(form, digest, a, s);
+  if (tp.sparse_threads == 512) return launch_pair_sparse_as<512, 1>(form, digest, a, s);
   switch (tp.pair_threads) {
     case 128:
       launch_pair_tiles_as<128>(form, digest, a, s);

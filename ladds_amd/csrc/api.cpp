@@ -115,7 +115,6 @@ struct ladds_ctx {
   void *scratch = nullptr;
   size_t scratch_bytes = 0;
   size_t tps_alloc = 0;
-  uint32_t *n_alive = nullptr;
   uint32_t grid_buckets_alloc = 0;
   size_t tile_sum_alloc = 0;
 
@@ -137,6 +136,8 @@ struct ladds_ctx {
   LoggedPair *h_log = nullptr;
   size_t h_log_cap = 0;
   void *h_x = nullptr;
+  uint32_t *h_tiles = nullptr;  // mapped, coherent: survivors per tile (compact_if_needed)
+  size_t h_tiles_alloc = 0;
   size_t h_x_bytes = 0;
   // The device pair log may hold entries of ladds_simulate not yet cleared.
   bool log_nonempty = false;
@@ -640,8 +641,8 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     else if (cap1 <= kSparseMost)
       set(mean < 200 ? 128 : (used >= 512 ? 256 : 512), 1, cap1);
     if (tp.sparse_threads && pair_sparse_lds_bytes(tp) > kPairTileLdsBytes) tp.sparse_threads = 0u;
-    // one workgroup does a plane whose records fit (64 scenarios of 1,024 to 65,536 objects:
-    // the fullest planes chunked in the sorting kernel 240 us per step, here 130)
+    // one workgroup does a plane whose records fit (47 scenarios of 1,024 to 65,536 objects, split:
+    // with the fullest planes chunked in the sorting kernel 239 us per step, here 115)
     if (tp.sparse_threads) tp.nchunk = 1;
   }
   // scratch arena for planes beyond the LDS capacity: every chunk of a plane sorts it
@@ -1098,21 +1099,35 @@ int capture_step_graph(ladds_ctx *ctx, int b, double burnup_r2, bool digest, hip
   return LADDS_OK;
 }
 
-int compact_if_needed(ladds_ctx *ctx) {
+// Removes the flagged objects (activity < 0; burn_r2 > 0: after flagging those with |r|^2
+// below it).  Waits for the count; where objects are removed, the compaction may still run
+// when it returns (ladds_ctx::pending).
+int compact_if_needed(ladds_ctx *ctx, double burn_r2 = 0.0) {
   if (ctx->n == 0) return LADDS_OK;
   const uint32_t ntiles = (uint32_t)((ctx->n + kCompactTile - 1) / kCompactTile);
-  if (!ctx->d_alt.rx) HIPCHK(ctx, alloc_objects(ctx->d_alt, ctx->cap));
-  DeviceObjects dst = ctx->d_alt;
-  dst.n = ctx->n;
-  hipError_t e = launch_count_alive(ctx->d, ctx->tile_sum, ntiles, ctx->stream);
-  if (e == hipSuccess)
-    e = timed(ctx, "compact",
-              [&] { return launch_compact(ctx->d, dst, ctx->tile_sum, ntiles, ctx->n_alive, ctx->stream); });
-  if (e != hipSuccess) return ctx->hipfail(e, "compaction launch");
-  uint32_t alive = 0;
-  HIPCHK(ctx, hipMemcpyAsync(&alive, ctx->n_alive, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+  if (ntiles > ctx->h_tiles_alloc) {
+    if (ctx->h_tiles) hipHostFree(ctx->h_tiles);
+    ctx->h_tiles = nullptr;
+    ctx->h_tiles_alloc = 0;
+    HIPCHK(ctx, hipHostMalloc(reinterpret_cast<void **>(&ctx->h_tiles), sizeof(uint32_t) * ntiles,
+                              hipHostMallocMapped | hipHostMallocCoherent));
+    ctx->h_tiles_alloc = ntiles;
+  }
+  uint32_t *host_sum = nullptr;
+  HIPCHK(ctx, hipHostGetDevicePointer(reinterpret_cast<void **>(&host_sum), ctx->h_tiles, 0));
+  HIPCHK(ctx, launch_count_alive(ctx->d, burn_r2, ctx->tile_sum, host_sum, ntiles, ctx->stream));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->pending = false;
+  size_t alive = 0;
+  for (uint32_t t = 0; t < ntiles; ++t) alive += ctx->h_tiles[t];
   if (alive != ctx->n) {
+    if (!ctx->d_alt.rx) HIPCHK(ctx, alloc_objects(ctx->d_alt, ctx->cap));
+    DeviceObjects dst = ctx->d_alt;
+    dst.n = ctx->n;
+    const hipError_t e =
+        timed(ctx, "compact", [&] { return launch_compact(ctx->d, dst, ctx->tile_sum, ntiles, ctx->stream); });
+    if (e != hipSuccess) return ctx->hipfail(e, "compaction launch");
+    ctx->pending = true;
     std::vector<int32_t> act;
     if (ctx->scen_off.size() > 2) {  // the flags of the pre-compaction arrays give the new offsets
       act.resize(ctx->n);
@@ -1132,6 +1147,8 @@ int compact_if_needed(ladds_ctx *ctx) {
       }
       ctx->scen_off = off;
       std::vector<double> rx(alive);
+      const int settled = settle(ctx);
+      if (settled != LADDS_OK) return settled;
       if (alive) HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * alive, hipMemcpyDeviceToHost));
       const int rc = setup_grid(ctx, alive, rx.data());
       if (rc != LADDS_OK) return rc;
@@ -1226,7 +1243,6 @@ int ladds_create(const ladds_config *cfg, ladds_ctx **out) {
       e = hipMemset(rb, 0, sizeof(DeviceReadback));
     }
   }
-  if (e == hipSuccess) e = dalloc(&ctx->n_alive, 1);
   if (e != hipSuccess) {
     ladds_destroy(ctx);
     return (e == hipErrorOutOfMemory) ? LADDS_E_NOMEM : LADDS_E_HIP;
@@ -1269,6 +1285,7 @@ int ladds_destroy(ladds_ctx *ctx) {
   if (ctx->h_rb) hipHostFree(ctx->h_rb);
   if (ctx->h_log) hipHostFree(ctx->h_log);
   if (ctx->h_x) hipHostFree(ctx->h_x);
+  if (ctx->h_tiles) hipHostFree(ctx->h_tiles);
   hipFree(ctx->d_spawn);
   if (ctx->stream2) hipStreamDestroy(ctx->stream2);
   if (ctx->stream3) hipStreamDestroy(ctx->stream3);
@@ -1280,7 +1297,6 @@ int ladds_destroy(ladds_ctx *ctx) {
   hipFree(ctx->start);
   hipFree(ctx->tile_sum);
   hipFree(ctx->rec);
-  hipFree(ctx->n_alive);
   hipFree(ctx->tps);
   hipFree(ctx->scratch);
   hipFree(ctx->arena_top);
@@ -2389,7 +2405,8 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
   if (sc.overflow) return ctx->fail(LADDS_E_OVERFLOW, "conjunction scan scratch arena exhausted");
   // burnt-up objects were flagged by the propagation; compaction only when there are some
   if (min_altitude_km > 0.0 && sc.burnups > 0) {
-    const int rc = compact_if_needed(ctx);
+    int rc = compact_if_needed(ctx);
+    if (rc == LADDS_OK) rc = settle(ctx);
     if (rc != LADDS_OK) return rc;
   }
   if (stats) {
@@ -2498,29 +2515,11 @@ int ladds_clear_log(ladds_ctx *ctx) {
 
 int ladds_delete_burnups(ladds_ctx *ctx, double min_altitude_km, size_t *removed) {
   if (!ctx) return LADDS_E_INVALID;
-  LADDS_SETTLE(ctx);
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const size_t before = ctx->n;
-  if (before) {
-    // mark, then compact: a zero-step propagation applies only the burn-up test
+  if (before) {  // (follows steps that ladds_propagate left running on the stream)
     const double r = min_altitude_km + kREarth;
-    std::vector<double> hx(before), hy(before), hz(before);
-    std::vector<int32_t> act(before);
-    HIPCHK(ctx, hipMemcpyAsync(hx.data(), ctx->d.rx, 8 * before, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(hy.data(), ctx->d.ry, 8 * before, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(hz.data(), ctx->d.rz, 8 * before, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(act.data(), ctx->d.activity, 4 * before, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    const double r2 = r * r;
-    for (size_t i = 0; i < before; ++i) {
-      double s = 0.0;
-      s += hx[i] * hx[i];
-      s += hy[i] * hy[i];
-      s += hz[i] * hz[i];
-      if (s < r2) act[i] = -1;
-    }
-    HIPCHK(ctx, hipMemcpyAsync(ctx->d.activity, act.data(), 4 * before, hipMemcpyHostToDevice, ctx->stream));
-    const int rc = compact_if_needed(ctx);
+    const int rc = compact_if_needed(ctx, r * r);
     if (rc != LADDS_OK) return rc;
   }
   if (removed) *removed = before - ctx->n;

@@ -70,10 +70,13 @@ inline double search_radius(int form, double cutoff_km) {
   return form == kFormFp64 ? cutoff_km : cutoff_km * (1.0 + 1e-5) + 0.1;
 }
 
-// Burn-up compaction: alive flags are activity >= 0.
-hipError_t launch_count_alive(const DeviceObjects &o, uint32_t *tile_sum, uint32_t ntiles, hipStream_t s);
+// Burn-up compaction: alive flags are activity >= 0 (burn_r2 > 0: set to -1 for |r|^2 below it
+// first).  The survivors per tile go to tile_sum and to host_sum (device address of mapped host
+// memory).
+hipError_t launch_count_alive(const DeviceObjects &o, double burn_r2, uint32_t *tile_sum, uint32_t *host_sum,
+                              uint32_t ntiles, hipStream_t s);
 hipError_t launch_compact(const DeviceObjects &src, const DeviceObjects &dst, const uint32_t *tile_sum,
-                          uint32_t ntiles, uint32_t *n_alive, hipStream_t s);
+                          uint32_t ntiles, hipStream_t s);
 
 constexpr uint32_t kCompactTile = 2048;
 

@@ -287,7 +287,7 @@ typedef struct ladds_tuning {
                          /* (ladds_config.tune_simulate: wall time per step)    */
   double default_us;     /* the same for the untuned default [us]               */
   int32_t tried;         /* configurations timed                                */
-  int32_t tile_size;     /* chosen objects per partition tile                   */
+  int32_t tile_size;     /* chosen objects per partition tile (4096: at most)   */
   int32_t chunks;        /* chosen workgroups per plane (dense planes)          */
   int32_t workgroups_per_cu; /* pair-kernel workgroups per CU its LDS is sized for */
   double plane_width_km; /* chosen cell length along x (plane width) [km]       */

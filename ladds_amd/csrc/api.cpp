@@ -463,7 +463,16 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     ctx->tile_sum_alloc = ts_need;
   }
   TileParams tp{};
-  tp.tile_size = (ctx->tune_tile == 4096 || ctx->tune_tile == 16384) ? (uint32_t)ctx->tune_tile : kPartitionTile;
+  // Tiles enough to spread the partition over the CUs, and few segments for the pair kernel to
+  // gather a plane from.  Partition + pair kernel, us, tiles of 1024 / 2048 / 4096 / 8192: 16,384
+  // objects (FP64) 19.2 / 19.9 / 23.0 / 27.8; 131,072 (FP64) 28.7 / 26.6 / 27.7 / 32.7; 262,144
+  // (split) 36.7 / 29.9 / 28.3 / 29.9; 1,000,000 (FP64) 83 / 66 / 62 / 57.  Scenarios have tiles of
+  // their own.  A tuning's 4096 is the most: its smaller ones are these.
+  const bool one = ctx->scen_off.size() <= 2;
+  tp.tile_size = n <= 32768 ? 1024u : n <= 131072 ? 2048u : n <= 524288 ? 4096u : kPartitionTile;
+  if (!one) tp.tile_size = kPartitionTile;
+  if (ctx->tune_tile == 4096) tp.tile_size = std::min(tp.tile_size, 4096u);
+  if (ctx->tune_tile == 8192 || ctx->tune_tile == 16384) tp.tile_size = (uint32_t)ctx->tune_tile;
   tp.ntiles = (uint32_t)std::max<size_t>(1, (n + tp.tile_size - 1) / tp.tile_size);
   tp.nscen = 1;
   if (tiles && ctx->scen_off.size() > 2) {
@@ -1828,7 +1837,8 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
   // tile, chunks, workgroups per CU, dispatch order, ensemble objects per plane (0: 64), row
   // height and bucket width in cells, persistent pair kernel, pair-scan streams (0: by form)}
   double cur_cell = base_cell, cur_fx = 1.0;
-  int cur[11] = {-1, (int)ctx->tiles.pair_threads, (int)ctx->tiles.tile_size, (int)ctx->tiles.nchunk, 0,
+  int cur[11] = {-1, (int)ctx->tiles.pair_threads, std::max(4096, (int)ctx->tiles.tile_size),
+                 (int)ctx->tiles.nchunk, 0,
                  ctx->tiles.plane_order ? 1 : 0, 0, ctx->tiles.half_rows ? 2 : 1, ctx->tiles.half_buckets ? 2 : 1,
                  0, 0};
   double default_us = 0.0;
@@ -1981,7 +1991,7 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
     out->plane_width_km = 1.0 / ctx->grid.inv_cell_x;
     out->plane_bits = (int32_t)(ctx->grid.by + ctx->grid.bz);
     out->pair_threads = (int32_t)ctx->tiles.pair_threads;
-    out->tile_size = (int32_t)ctx->tiles.tile_size;
+    out->tile_size = std::max<int32_t>(4096, (int32_t)ctx->tiles.tile_size);  // (set_tuning's range; see setup_grid)
     out->chunks = (int32_t)ctx->tiles.nchunk;
     out->workgroups_per_cu = (int32_t)ctx->tune_wgs;
     out->plane_order = (int32_t)ctx->tune_order;

@@ -1015,6 +1015,12 @@ hipError_t launch_tile_partition_as(const DeviceObjects &o, const uint32_t *keys
                                     uint32_t *tps, uint32_t *arena_top, hipStream_t s, size_t stage_bytes) {
   REC *out = static_cast<REC *>(items);
   switch (tp.tile_size) {
+    case 1024:
+      launch_partition_items<REC, 1>(o, keys, tp, out, tps, arena_top, s, stage_bytes);
+      break;
+    case 2048:
+      launch_partition_items<REC, 2>(o, keys, tp, out, tps, arena_top, s, stage_bytes);
+      break;
     case 4096:
       launch_partition_items<REC, 4>(o, keys, tp, out, tps, arena_top, s, stage_bytes);
       break;
@@ -1088,9 +1094,13 @@ hipError_t configure_tile_kernels() {
   auto set = [&](const void *f) {
     if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, max_lds);
   };
+  set(reinterpret_cast<const void *>(&k_tile_partition<RecordF64, 1>));
+  set(reinterpret_cast<const void *>(&k_tile_partition<RecordF64, 2>));
   set(reinterpret_cast<const void *>(&k_tile_partition<RecordF64, 4>));
   set(reinterpret_cast<const void *>(&k_tile_partition<RecordF64, 8>));
   set(reinterpret_cast<const void *>(&k_tile_partition<RecordF64, 16>));
+  set(reinterpret_cast<const void *>(&k_tile_partition<RecordF32, 1>));
+  set(reinterpret_cast<const void *>(&k_tile_partition<RecordF32, 2>));
   set(reinterpret_cast<const void *>(&k_tile_partition<RecordF32, 4>));
   set(reinterpret_cast<const void *>(&k_tile_partition<RecordF32, 8>));
   set(reinterpret_cast<const void *>(&k_tile_partition<RecordF32, 16>));

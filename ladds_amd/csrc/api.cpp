@@ -1082,23 +1082,46 @@ int pair_streams(const ladds_ctx *ctx) {
   return ctx->form == kFormFp64 ? 1 : 2;
 }
 
-// Software-pipelined step graph for state buffer b: the pair scan of the state in b (on a
-// forked branch) runs beside the propagation of b into 1 - b and its partition (one step
-// ahead, environment step + 1); then the device step advances.  Two graphs, b = 0 and 1,
-// alternate.  Nothing is memset inside: the partition kernel resets its scratch arena.
-int capture_step_graph(ladds_ctx *ctx, int b, double burnup_r2, bool digest, hipGraphExec_t *exec) {
+// Steps of the longer step graph (even): its launch and end are paid once in eight steps (us per
+// step at 16,384 objects, FP64: 45 with one forked step per graph, 24 with one serial step, 19 with
+// eight; 16 steps 19.4; 1,000,000 split: 71 forked, 65 with eight forked).
+constexpr int kGraphSteps = 8;
+// Up to here a graph's kernels follow each other: the fork and the join cost more than the pair
+// scan hides (eight steps, us per step, serial against forked: 262,144 FP64 38 and 45; 400,000
+// split 46 and 41.5).
+constexpr size_t kSerialGraphObjects = 262144;
+// Up to here the eager loop, too, puts the three kernels of a step on one stream: the events
+// between the streams cost more than the overlap gains, and make the time depend on how the
+// streams are scheduled (us per step, serial against overlapped in the better and the worse
+// runs: 16,384 FP64 19.5 against 23 to 36; 65,521 split 23.4, 23 to 35; 131,072 FP64 28.5, 26 to 37;
+// 200,000 split 30.8, 26 to 32). With a detection in every third step or fewer the streams stay:
+// the other steps are one launch (65,521 objects, 80 km, every third: overlapped 10, serial 12.6).
+constexpr size_t kSerialObjects = 131072;
+
+// Step graph of `steps` steps from state buffer b.  Each step: the pair scan of the state in b,
+// the propagation of b into 1 - b (one step ahead, environment step + 1) and its partition; after
+// the last the device step advances.  `fork`: the pair scan on a branch beside the other two,
+// joined at the end of the step.  Two graphs, b = 0 and 1, alternate.  Nothing is memset inside:
+// the partition kernel resets its scratch arena.
+int capture_step_graph(ladds_ctx *ctx, int b, int steps, bool fork, double burnup_r2, bool digest,
+                       hipGraphExec_t *exec) {
   *exec = nullptr;
   hipGraph_t graph = nullptr;
   HIPCHK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
   int rc = LADDS_OK;
-  hipError_t e = hipEventRecord(ctx->ev_part[0], ctx->stream);  // fork
-  if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream2, ctx->ev_part[0], 0);
-  if (e == hipSuccess)
-    rc = launch_pairs_of(ctx, b, ctx->cfg.dt, digest, 0, ctx->d_step, ctx->stream2, ctx->protected_objects ? 1 : 0);
-  if (e == hipSuccess && rc == LADDS_OK) rc = launch_prop_part(ctx, b, 0, 1, true, burnup_r2, ctx->d_step, 1u);
-  if (e == hipSuccess && rc == LADDS_OK) e = hipEventRecord(ctx->ev_pair[0], ctx->stream2);  // join
-  if (e == hipSuccess && rc == LADDS_OK) e = hipStreamWaitEvent(ctx->stream, ctx->ev_pair[0], 0);
-  if (e == hipSuccess && rc == LADDS_OK) e = launch_advance_step(ctx->d_step, ctx->stream);
+  hipError_t e = hipSuccess;
+  hipStream_t ps = fork ? ctx->stream2 : ctx->stream;
+  for (int k = 0; k < steps && rc == LADDS_OK && e == hipSuccess; ++k, b = 1 - b) {
+    if (fork) e = hipEventRecord(ctx->ev_part[0], ctx->stream);
+    if (fork && e == hipSuccess) e = hipStreamWaitEvent(ps, ctx->ev_part[0], 0);
+    if (e == hipSuccess)
+      rc = launch_pairs_of(ctx, b, ctx->cfg.dt, digest, (uint64_t)k, ctx->d_step, ps, ctx->protected_objects ? 1 : 0);
+    if (e == hipSuccess && rc == LADDS_OK)
+      rc = launch_prop_part(ctx, b, 0, 1, true, burnup_r2, ctx->d_step, (uint32_t)k + 1u);
+    if (fork && e == hipSuccess && rc == LADDS_OK) e = hipEventRecord(ctx->ev_pair[0], ps);  // join
+    if (fork && e == hipSuccess && rc == LADDS_OK) e = hipStreamWaitEvent(ctx->stream, ctx->ev_pair[0], 0);
+  }
+  if (e == hipSuccess && rc == LADDS_OK) e = launch_advance_step(ctx->d_step, (uint32_t)steps, ctx->stream);
   const hipError_t ec = hipStreamEndCapture(ctx->stream, &graph);
   if (rc == LADDS_OK && e == hipSuccess) e = ec;
   if (rc == LADDS_OK && e == hipSuccess) e = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
@@ -2210,7 +2233,8 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
   // and stream4 with pair_streams 2) of consecutive steps: see overlapped_iteration.
   const bool use_graph = ctx->cfg.step_graph != 0 && tpcd == 1 && ctx->variant == kVariantPlaneTiles &&
                          !ctx->profiling && ctx->n > 0 && nsteps > 0;
-  const bool use_overlap = !use_graph && ctx->variant == kVariantPlaneTiles && ctx->n > 0 && nsteps > 0;
+  const bool use_overlap = !use_graph && ctx->variant == kVariantPlaneTiles && ctx->n > 0 && nsteps > 0 &&
+                           (ctx->n > kSerialObjects || tpcd > 2);
   // The eager loop's first iteration runs on stream2 (overlapped_iteration's `fill`), and so
   // does what precedes it here (counter reset, spawn state, environments), after anything
   // still queued on the context's stream.
@@ -2250,16 +2274,17 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
     const int rc = ensure_overlap_buffers(ctx, use_graph ? 2 : nbuf);
     if (rc != LADDS_OK) return rc;
   }
-  hipGraphExec_t graphs[2] = {nullptr, nullptr};
+  hipGraphExec_t graphs[4] = {nullptr, nullptr, nullptr, nullptr};  // one step from buffer 0, 1; several steps
   auto drop_graphs = [&] {
     for (hipGraphExec_t &g : graphs)
       if (g) hipGraphExecDestroy(g);
   };
+  const bool fork = ctx->n > kSerialGraphObjects;
   if (use_graph) {
     if (!ctx->d_step) HIPCHK(ctx, dalloc(&ctx->d_step, 1));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     for (int b = 0; b < 2; ++b) {
-      const int rc = capture_step_graph(ctx, b, burnup_r2, digest, &graphs[b]);
+      const int rc = capture_step_graph(ctx, b, 1, fork, burnup_r2, digest, &graphs[b]);
       if (rc != LADDS_OK) {
         drop_graphs();
         return rc;
@@ -2289,7 +2314,15 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
       hipError_t e = launch_set_step(ctx->d_step, (uint32_t)env_off, base - (uint64_t)env_off, ctx->stream);
       if (e == hipSuccess) rc = launch_prop_part(ctx, cur, env_off, 1, true, burnup_r2, nullptr, 0);
       cur = 1 - cur;
-      for (int j = 0; j + 1 < seg && rc == LADDS_OK && e == hipSuccess; ++j) {
+      int j = 0;
+      if (seg > 4 * kGraphSteps) {
+        hipGraphExec_t &several = graphs[2 + cur];  // (an even number of steps ends in the buffer it began with)
+        if (!several && e == hipSuccess && rc == LADDS_OK)
+          rc = capture_step_graph(ctx, cur, kGraphSteps, fork, burnup_r2, digest, &several);
+        for (; j + kGraphSteps < seg && rc == LADDS_OK && e == hipSuccess; j += kGraphSteps)
+          e = hipGraphLaunch(several, ctx->stream);
+      }
+      for (; j + 1 < seg && rc == LADDS_OK && e == hipSuccess; ++j) {
         e = hipGraphLaunch(graphs[cur], ctx->stream);
         cur = 1 - cur;
       }

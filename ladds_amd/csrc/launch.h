@@ -17,7 +17,7 @@ hipError_t launch_propagate(int form, const DeviceObjects &o, const SubstepEnv<d
                             unsigned long long *burnups = nullptr);
 // Graph replay bookkeeping: set the step position, advance it by one step.
 hipError_t launch_set_step(StepState *st, uint32_t step, uint64_t iter_base, hipStream_t stream);
-hipError_t launch_advance_step(StepState *st, hipStream_t stream);
+hipError_t launch_advance_step(StepState *st, uint32_t steps, hipStream_t stream);
 // Copies `words` 8-byte words from device memory to mapped host memory (one workgroup).
 hipError_t launch_publish(const unsigned long long *src, unsigned long long *dst, int words, hipStream_t stream);
 

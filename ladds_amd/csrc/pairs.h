@@ -193,11 +193,11 @@ struct PairSink {
   unsigned long long *log_count;
   ScanCounters *counters;
   uint64_t iteration;
-  const StepState *step_state;  // non-null (graph replay): iteration = iter_base + step
+  const StepState *step_state;  // non-null (graph replay): iteration counts from iter_base + step
 };
 
 __device__ __forceinline__ unsigned long long sink_iteration(const PairSink &a) {
-  return a.step_state ? a.step_state->iter_base + a.step_state->step : a.iteration;
+  return a.step_state ? a.step_state->iter_base + a.step_state->step + a.iteration : a.iteration;
 }
 
 struct ScanAcc {

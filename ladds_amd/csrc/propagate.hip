@@ -240,8 +240,8 @@ __global__ void k_set_step(StepState *st, uint32_t step, uint64_t iter_base) {
   }
 }
 
-__global__ void k_advance_step(StepState *st) {
-  if (threadIdx.x == 0) st->step += 1u;
+__global__ void k_advance_step(StepState *st, uint32_t steps) {
+  if (threadIdx.x == 0) st->step += steps;
 }
 
 hipError_t launch_set_step(StepState *st, uint32_t step, uint64_t iter_base, hipStream_t stream) {
@@ -249,8 +249,8 @@ hipError_t launch_set_step(StepState *st, uint32_t step, uint64_t iter_base, hip
   return hipGetLastError();
 }
 
-hipError_t launch_advance_step(StepState *st, hipStream_t stream) {
-  hipLaunchKernelGGL(k_advance_step, dim3(1), dim3(64), 0, stream, st);
+hipError_t launch_advance_step(StepState *st, uint32_t steps, hipStream_t stream) {
+  hipLaunchKernelGGL(k_advance_step, dim3(1), dim3(64), 0, stream, st, steps);
   return hipGetLastError();
 }
 

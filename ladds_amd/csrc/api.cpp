@@ -1000,6 +1000,13 @@ int launch_pairs_of(ladds_ctx *ctx, int b, double dt_interp, bool digest, uint64
 // us per step, 20-step calls 103.9 -> 102.0).
 constexpr size_t kPipelineStageBytes = 64 * 1024;
 
+// Up to this many objects the partition of a short propagation follows it on its stream: the hop
+// to the third stream costs more than the partition (us per step, behind it against beside the
+// next propagation: 65,521 objects, split, 16 to 20 against 23 to 35; 200,000 split 28 against 26
+// to 32; 65,521, 80 km, a detection every third step, 8.7 against 11; every tenth 4.1 against 3.7).
+constexpr size_t kPartBehindObjects = 262144;
+constexpr int kPartBehindSteps = 4;
+
 // One iteration of the eager overlapped loop: propagate buffer `cur` into nxt = cur + 1
 // (mod nbuf) on `stream` and, when `detect`, partition nxt on `stream3` once the propagation
 // is done; its pair scan (issue_scan) is queued by the next iteration.  Buffer nxt was last
@@ -1038,9 +1045,10 @@ int overlapped_iteration(ladds_ctx *ctx, int nbuf, int cur, bool pending_next, s
   }
   int rc = launch_prop_into(ctx, cur, nxt, env_offset, nsteps, detect, burnup_r2, nullptr, 0);
   if (rc != LADDS_OK || !detect) return rc;
-  rc = follow(ctx, ctx->ev_prop[nxt], ctx->stream, ctx->stream3);
-  if (rc == LADDS_OK) rc = launch_part_of(ctx, nxt, ctx->stream3, stage);
-  if (rc == LADDS_OK) HIPCHK(ctx, hipEventRecord(ctx->ev_part[nxt], ctx->stream3));
+  hipStream_t part = ctx->n <= kPartBehindObjects && nsteps <= kPartBehindSteps ? ctx->stream : ctx->stream3;
+  if (part != ctx->stream) rc = follow(ctx, ctx->ev_prop[nxt], ctx->stream, part);
+  if (rc == LADDS_OK) rc = launch_part_of(ctx, nxt, part, stage);
+  if (rc == LADDS_OK) HIPCHK(ctx, hipEventRecord(ctx->ev_part[nxt], part));
   return rc;
 }
 
@@ -1090,13 +1098,11 @@ constexpr int kGraphSteps = 8;
 // scan hides (eight steps, us per step, serial against forked: 262,144 FP64 38 and 45; 400,000
 // split 46 and 41.5).
 constexpr size_t kSerialGraphObjects = 262144;
-// Up to here the eager loop, too, puts the three kernels of a step on one stream: the events
-// between the streams cost more than the overlap gains, and make the time depend on how the
-// streams are scheduled (us per step, serial against overlapped in the better and the worse
-// runs: 16,384 FP64 19.5 against 23 to 36; 65,521 split 23.4, 23 to 35; 131,072 FP64 28.5, 26 to 37;
-// 200,000 split 30.8, 26 to 32). With a detection in every third step or fewer the streams stay:
-// the other steps are one launch (65,521 objects, 80 km, every third: overlapped 10, serial 12.6).
-constexpr size_t kSerialObjects = 131072;
+// Up to here the eager loop, too, puts the three kernels of a step on one stream (us per step,
+// serial against overlapped with the partition behind the propagation: 4,096 objects, FP64, 17.8
+// against 20.2; 16,384 19.5 and 22.5; 32,768 21.3, 19 to 23; 65,521 split 22.0, 16 to 20). With a
+// detection in every third step or fewer the streams stay: the other steps are one launch.
+constexpr size_t kSerialObjects = 32768;
 
 // Step graph of `steps` steps from state buffer b.  Each step: the pair scan of the state in b,
 // the propagation of b into 1 - b (one step ahead, environment step + 1) and its partition; after

@@ -46,10 +46,11 @@ struct PropagateArgs {
 // STAGED: the environments go through LDS (EnvStage).  With one wavefront per SIMD or less the
 // scalar loads of environments that no other wavefront of the XCD has read yet took half of
 // a step (4,099 objects, FP64, components branched over: 3.83 us per step, 2.05 staged).
-// Larger populations keep the 5.7 KB of LDS free: beside the pair kernel a propagation workgroup
-// then finds room on every CU (1,048,576 objects, split: 108.2 ms per 1,440 steps of the
-// simulation loop staged, 102.2 without).
-constexpr size_t kStagedObjects = 32768;
+// With four (65,521 objects, ten steps a launch, 400 steps: 2.20 ms, 1.89 staged; 250,007, 1000
+// steps: 6.14 and 5.97 ms) it still gains a little. Larger populations keep the 5.7 KB of LDS
+// free for the pair kernel beside them (1,048,576 objects, split, 1,440 steps of the simulation
+// loop: 95.4 ms staged, 94.0 without).
+constexpr size_t kStagedObjects = 262144;
 
 template <int FORM, bool STAGED>
 __global__ __launch_bounds__(256) void k_propagate(PropagateArgs a) {

@@ -29,7 +29,7 @@ def _run(pop, precision, graph, calls, tpcd=1):
 @pytest.mark.parametrize("precision", [la.FP64, la.SPLIT])
 @pytest.mark.parametrize("n,calls", [
     (20000, [33, 34, 41, 8, 50]),   # serial graphs: at, above and below the several-step graph's least length
-    (131073, [40, 35]),             # the eager loop overlaps, the graphs are serial
+    (40001, [40, 35]),              # the eager loop overlaps, the graphs are serial
     (262145, [49, 34]),             # both overlap
 ])
 def test_graphs_match_the_eager_loop(precision, n, calls):
@@ -43,11 +43,11 @@ def test_graphs_match_the_eager_loop(precision, n, calls):
 
 
 @pytest.mark.parametrize("precision", [la.FP64, la.SPLIT])
-@pytest.mark.parametrize("tpcd", [1, 2, 3])
-def test_serial_and_overlapped_loops_agree(precision, tpcd):
-    """131,072 objects run on one stream, 131,073 overlapped: the last one, far from all others,
-    changes nothing else."""
-    n = 131073
+@pytest.mark.parametrize("tpcd", [1, 2, 3, 5])
+@pytest.mark.parametrize("n", [32769, 262145])
+def test_serial_and_overlapped_loops_agree(precision, tpcd, n):
+    """32,768 objects run on one stream, 32,769 overlapped (262,144 and 262,145: the partition behind
+    the propagation, and beside the next): the last one, far from all others, changes nothing else."""
     pop = la.generate_population(1, 12, n)
     r = pop.r()
     far = 60000.0 / np.linalg.norm(r[-1])

@@ -292,7 +292,7 @@ typedef struct ladds_tuning {
   int32_t workgroups_per_cu; /* pair-kernel workgroups per CU its LDS is sized for */
   double plane_width_km; /* chosen cell length along x (plane width) [km]       */
   int32_t plane_order;   /* pair-kernel dispatch: 0 plane order, 1 heaviest planes first */
-  int32_t ensemble_plane_objects; /* ensembles: objects per x-plane (0: the default 64)   */
+  int32_t ensemble_plane_objects; /* ensembles: objects per x-plane (0: the default 256)  */
   int32_t row_cells;     /* bucket row height along y in cells: 1 (an object scans three */
                          /* rows of the next plane) or 2 (two rows, on the side of the   */
                          /* half of its row it lies in); 0 is read as 1                  */

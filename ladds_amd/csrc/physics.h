@@ -255,10 +255,12 @@ __device__ __forceinline__ void acceleration(double x, double y, double z, doubl
   const double inv_r = rsqrt64(r2);
   const double inv_r2 = inv_r * inv_r;
   const double inv_r3 = inv_r2 * inv_r;
-  const double fk = ((mask & kKepBit) ? -kMuEarth : 0.0) * inv_r3;
-  ax = fk * x;
-  ay = fk * y;
-  az = fk * z;
+  // (chosen, not multiplied by 0: without this force an object at the origin, or infinitely far, has none)
+  const bool kepler = (mask & kKepBit) != 0u;
+  const double fk = -kMuEarth * inv_r3;
+  ax = kepler ? fk * x : 0.0;
+  ay = kepler ? fk * y : 0.0;
+  az = kepler ? fk * z : 0.0;
   constexpr bool j2_64 = (FORM != kFormSplitAll32);
   constexpr bool tess_64 = (FORM != kFormSplitAll32);
   const double inv_r5 = inv_r3 * inv_r2;

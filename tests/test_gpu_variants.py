@@ -61,3 +61,23 @@ def test_adjoint_forward_variants_agree(every):
 
     for a, b in zip(run(pop), run(_take(pop, EDGE))):
         assert np.array_equal(a[:EDGE], b)
+
+
+@pytest.mark.parametrize("precision", [la.FP64, la.SPLIT, la.SPLIT_ALL32])
+@pytest.mark.parametrize("n", [70, EDGE + 70])
+def test_no_force_where_none_is_asked_for(precision, n):
+    """Without components an object moves along its velocity, also at the origin and infinitely far,
+    where the powers of the radius are not finite."""
+    r = np.zeros((n, 3))
+    r[:, 0] = np.arange(n)
+    r[3] = [np.inf, 0.0, 0.0]
+    r[5] = [0.0, 1.0e300, -1.0e-200]
+    v = np.zeros_like(r)
+    v[:, 2] = np.arange(n) * 1.0e-3
+    with la.Engine(la.EngineConfig(precision=precision, components=0, cutoff_km=10.0, dt=1.0)) as eng:
+        eng.set_objects(rx=r[:, 0], ry=r[:, 1], rz=r[:, 2], vx=v[:, 0], vy=v[:, 1], vz=v[:, 2], radius_m=np.ones(n))
+        eng.propagate(3)
+        r1, v1 = eng.state()
+    assert np.array_equal(v1, v)
+    np.testing.assert_array_equal(r1[:, :2], r[:, :2])
+    np.testing.assert_allclose(r1[:, 2], r[:, 2] + 3.0 * v[:, 2], rtol=1e-14, atol=1e-14)

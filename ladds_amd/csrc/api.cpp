@@ -1681,22 +1681,6 @@ int ladds_propagate(ladds_ctx *ctx, int nsteps) {
   return LADDS_OK;
 }
 
-static int run_detection_sync(ladds_ctx *ctx, double dt_interp, bool digest, ScanCounters *out_counters,
-                              uint64_t *entries) {
-  HIPCHK(ctx, hipMemsetAsync(ctx->counters, 0, sizeof(ScanCounters), ctx->stream));
-  HIPCHK(ctx, hipMemsetAsync(ctx->log_count, 0, sizeof(unsigned long long), ctx->stream));
-  int rc = launch_detection(ctx, ctx->keys_valid, dt_interp, digest, 0);
-  if (rc != LADDS_OK) return rc;
-  unsigned long long cnt = 0;
-  HIPCHK(ctx, hipMemcpyAsync(out_counters, ctx->counters, sizeof(ScanCounters), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipMemcpyAsync(&cnt, ctx->log_count, sizeof(cnt), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  ctx->pending = false;
-  *entries = cnt;
-  if (out_counters->overflow) return ctx->fail(LADDS_E_OVERFLOW, "conjunction scan scratch arena exhausted");
-  return LADDS_OK;
-}
-
 // Device time of one detection (keys, partition, pair scan in digest mode) on the
 // current state: the minimum over `reps` runs after one warm-up run.
 // Smallest relative gain for which the autotuner moves to a candidate shape.
@@ -2107,16 +2091,21 @@ int ladds_conjunctions(ladds_ctx *ctx, double dt_interp, ladds_pair *hits, size_
     int rc = launch_detection(ctx, ctx->keys_valid, dt_interp, false, 0);
     if (rc != LADDS_OK) return rc;
     if (!ctx->h_log) {
-      HIPCHK(ctx, hipHostMalloc(reinterpret_cast<void **>(&ctx->h_log), sizeof(LoggedPair) * 4096, 0));
+      HIPCHK(ctx, hipHostMalloc(reinterpret_cast<void **>(&ctx->h_log), sizeof(LoggedPair) * 4096,
+                                hipHostMallocMapped | hipHostMallocCoherent));
       ctx->h_log_cap = 4096;
     }
     // the first 256 entries come back with the counters (a call that finds more copies the
     // rest after the first synchronisation)
     const size_t staged = std::min<size_t>({ctx->h_log_cap, ctx->log_cap, 256});
-    HIPCHK(ctx, hipMemcpyAsync(&ctx->h_rb->sc, ctx->counters, sizeof(DeviceReadback), hipMemcpyDeviceToHost,
-                               ctx->stream));  // counters and log count
-    HIPCHK(ctx, hipMemcpyAsync(ctx->h_log, ctx->log, sizeof(LoggedPair) * staged, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipMemsetAsync(ctx->log_count, 0, sizeof(unsigned long long), ctx->stream));
+    LoggedPair *host_log = nullptr;
+    HIPCHK(ctx, hipHostGetDevicePointer(reinterpret_cast<void **>(&host_log), ctx->h_log, 0));
+    // counters, log count and those entries in one launch (two copies and a fill before it:
+    // 16,384 objects, a step with detection, 68 -> 53 us, 100,003 97 -> 78)
+    HIPCHK(ctx, launch_publish_log(reinterpret_cast<const unsigned long long *>(ctx->counters),
+                                   reinterpret_cast<unsigned long long *>(&ctx->d_rb_host->sc),
+                                   (int)(sizeof(DeviceReadback) / 8), ctx->log_count, ctx->log, host_log,
+                                   (uint32_t)staged, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     ctx->pending = false;
     if (ctx->h_rb->sc.overflow) return ctx->fail(LADDS_E_OVERFLOW, "conjunction scan scratch arena exhausted");
@@ -2131,7 +2120,8 @@ int ladds_conjunctions(ladds_ctx *ctx, double dt_interp, ladds_pair *hits, size_
         size_t want = ctx->h_log_cap;
         while (want < entries) want *= 2;
         LoggedPair *bigger = nullptr;
-        HIPCHK(ctx, hipHostMalloc(reinterpret_cast<void **>(&bigger), sizeof(LoggedPair) * want, 0));
+        HIPCHK(ctx, hipHostMalloc(reinterpret_cast<void **>(&bigger), sizeof(LoggedPair) * want,
+                                  hipHostMallocMapped | hipHostMallocCoherent));
         std::memcpy(bigger, ctx->h_log, sizeof(LoggedPair) * staged);
         hipHostFree(ctx->h_log);
         ctx->h_log = bigger;
@@ -2202,15 +2192,18 @@ int ladds_conjunction_digest(ladds_ctx *ctx, double dt_interp, uint64_t *n, uint
   digest[0] = digest[1] = edigest[0] = edigest[1] = 0;
   if (ctx->n < 2) return LADDS_OK;
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  ScanCounters sc{};
-  uint64_t entries = 0;
-  unsigned long long saved = 0;
-  HIPCHK(ctx, hipMemcpyAsync(&saved, ctx->log_count, sizeof(saved), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  const int rc = run_detection_sync(ctx, dt_interp, true, &sc, &entries);
-  HIPCHK(ctx, hipMemcpyAsync(ctx->log_count, &saved, sizeof(saved), hipMemcpyHostToDevice, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  // digest output leaves the pair log and its count alone; one synchronisation
+  HIPCHK(ctx, hipMemsetAsync(ctx->counters, 0, sizeof(ScanCounters), ctx->stream));
+  const int rc = launch_detection(ctx, ctx->keys_valid, dt_interp, true, 0);
   if (rc != LADDS_OK) return rc;
+  static_assert(sizeof(ScanCounters) % 8 == 0, "whole words");
+  HIPCHK(ctx, launch_publish(reinterpret_cast<const unsigned long long *>(ctx->counters),
+                             reinterpret_cast<unsigned long long *>(&ctx->d_rb_host->sc),
+                             (int)(sizeof(ScanCounters) / 8), ctx->stream));
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  ctx->pending = false;
+  const ScanCounters sc = ctx->h_rb->sc;
+  if (sc.overflow) return ctx->fail(LADDS_E_OVERFLOW, "conjunction scan scratch arena exhausted");
   *n = sc.hits;
   *ne = sc.evaded;
   digest[0] = sc.digest[0];

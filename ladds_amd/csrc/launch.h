@@ -20,6 +20,11 @@ hipError_t launch_set_step(StepState *st, uint32_t step, uint64_t iter_base, hip
 hipError_t launch_advance_step(StepState *st, uint32_t steps, hipStream_t stream);
 // Copies `words` 8-byte words from device memory to mapped host memory (one workgroup).
 hipError_t launch_publish(const unsigned long long *src, unsigned long long *dst, int words, hipStream_t stream);
+// As launch_publish, then the first min(*log_count, most) entries of the log to host_log, and
+// *log_count (a word of src) reset.
+hipError_t launch_publish_log(const unsigned long long *src, unsigned long long *dst, int words,
+                              unsigned long long *log_count, const LoggedPair *log, LoggedPair *host_log,
+                              uint32_t most, hipStream_t stream);
 
 hipError_t launch_bin_count(int form, const DeviceObjects &o, const GridParams &g, uint32_t *count, uint32_t *slot,
                             hipStream_t s);

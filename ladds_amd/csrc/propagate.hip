@@ -261,6 +261,29 @@ __global__ void k_publish(const unsigned long long *src, unsigned long long *dst
   for (int k = threadIdx.x; k < words; k += blockDim.x) dst[k] = src[k];
 }
 
+// The same with the first entries of the pair log behind the counters: min(*log_count, `most`)
+// entries of `entry_words` words each; *log_count (one of the published words) is reset.
+__global__ void k_publish_log(const unsigned long long *src, unsigned long long *dst, int words,
+                              unsigned long long *log_count, const unsigned long long *log,
+                              unsigned long long *host_log, uint32_t most, uint32_t entry_words) {
+  const unsigned long long cnt = *log_count;
+  for (int k = threadIdx.x; k < words; k += blockDim.x) dst[k] = src[k];
+  const uint32_t n = (cnt < most ? (uint32_t)cnt : most) * entry_words;
+  for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) host_log[k] = log[k];
+  __syncthreads();  // every wavefront has read the count
+  if (threadIdx.x == 0) *log_count = 0ull;
+}
+
+hipError_t launch_publish_log(const unsigned long long *src, unsigned long long *dst, int words,
+                              unsigned long long *log_count, const LoggedPair *log, LoggedPair *host_log,
+                              uint32_t most, hipStream_t stream) {
+  static_assert(sizeof(LoggedPair) % 8 == 0, "whole words");
+  hipLaunchKernelGGL(k_publish_log, dim3(1), dim3(256), 0, stream, src, dst, words, log_count,
+                     reinterpret_cast<const unsigned long long *>(log),
+                     reinterpret_cast<unsigned long long *>(host_log), most, (uint32_t)(sizeof(LoggedPair) / 8));
+  return hipGetLastError();
+}
+
 hipError_t launch_publish(const unsigned long long *src, unsigned long long *dst, int words, hipStream_t stream) {
   hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, stream, src, dst, words);
   return hipGetLastError();

@@ -46,3 +46,29 @@ def test_removal_behind_a_step(precision, n, low):
             eng.propagate(1)
             assert eng.delete_burnups(1.0e6) == keep.size and eng.n == 0
         assert eng.delete_burnups(150.0) == 0
+
+
+@pytest.mark.parametrize("pairs", [0, 1, 255, 256, 257, 4097])
+def test_pair_lists_around_the_staged_entries(pairs):
+    """As many conjunctions as come back with the counters, one fewer and more; a digest between a
+    simulation and its fetch leaves the log alone."""
+    r = np.zeros((2 * pairs + 4, 3))
+    r[:, 0] = np.arange(len(r)) // 2 * 50.0
+    r[1::2, 1] = 0.5
+    r[2 * pairs:, 1] += 1000.0 * np.arange(4)
+    v = np.zeros_like(r)
+    v[:, 2] = np.linspace(0.0, 1e-3, len(r))
+    with la.Engine(la.EngineConfig(dt=10.0, components=0, cutoff_km=10.0, threshold_mode=la.THRESHOLD_ABSOLUTE,
+                                   threshold_km=5.0, log_capacity=8192)) as eng:
+        eng.set_objects(rx=r[:, 0], ry=r[:, 1], rz=r[:, 2], vx=v[:, 0], vy=v[:, 1], vz=v[:, 2],
+                        radius_m=np.ones(len(r)))
+        for _ in range(2):
+            hits, evaded = eng.conjunctions()
+            hits = ol.sort_pairs(hits)
+            assert len(evaded) == 0
+            assert hits["id_a"].tolist() == list(range(0, 2 * pairs, 2))
+            assert hits["id_b"].tolist() == list(range(1, 2 * pairs, 2))
+        s = eng.simulate(1, first_iteration=0, tpcd=1)
+        n, digest, _, _ = eng.conjunction_digest()
+        assert n == s["collisions"] == len(eng.fetch_log()) == pairs
+        assert digest == ol.digest(hits)

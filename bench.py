@@ -46,7 +46,8 @@ BYTES = {
     "propagate": {"fp64": 96 + 16 + 4 + 4, "split": 96 + 12 + 4 + 4},
     # keys read (4) + r read (24) + record write (32 | 16)
     "tile_partition": {"fp64": 4 + 24 + 32, "split": 4 + 24 + 16},
-    # every record read once for its own plane and once as the next plane of the plane below
+    # every record read for its own plane and as the next plane of the group below (two planes a
+    # workgroup: half of them twice from memory; counted twice)
     "pair_tiles": {"fp64": 2 * 32, "split": 2 * 16},
     # r read (24) + slot read (4) + bucket start (4) + record write (32 | 16) + index write (4)
     "bin_scatter": {"fp64": 24 + 4 + 4 + 32 + 4, "split": 24 + 4 + 4 + 16 + 4},
@@ -56,28 +57,25 @@ BYTES = {
 
 
 # HBM bytes per launch at 1,048,576 objects (read + write), measured with rocprofv3
-# FETCH_SIZE / WRITE_SIZE scaled by a 256 MiB copy kernel, on the plane-tile shape the
-# autotuner picks for this workload (FP64: 512-thread pair workgroups, 4,096-object tiles;
-# split: 256 threads, 8,192-object tiles; both: buckets of 2 x 2 cells); the runs and the
-# commands are in
-# profiles/hbm_traffic_1M_full_model.md.
+# FETCH_SIZE / WRITE_SIZE scaled by a 256 MiB copy kernel, on the default shape (sparse pair
+# kernel, 8,192-object tiles); the commands are in profiles/kernels_timed_cases.md.
 # FP64 and FP32 VALU flops per object-step of the propagation kernel (full force model),
 # from rocprofv3 SQ_INSTS_VALU_FLOPS_{FP64,FP32} (+ the _TRANS counters), per wavefront
 # instruction and lane, on the 1M-object workload.
 MEASURED_FLOPS_PER_OBJECT = {
-    ("propagate", "fp64"): (794.0 + 15.0, 0.0),
-    ("propagate", "split"): (551.0 + 6.0, 249.0 + 12.0),
+    ("propagate", "fp64"): (663.0 + 12.0, 0.0),
+    ("propagate", "split"): (477.0 + 6.0, 249.0 + 12.0),
 }
 FP64_PEAK_TFLOPS = 78.6   # MI355X vector FP64
 FP32_PEAK_TFLOPS = 157.3  # MI355X vector FP32 (non-packed issue is half of this)
 
 MEASURED_TRAFFIC_1M = {
-    ("propagate", "fp64"): (71.47 + 54.65) * 1e6,
-    ("propagate", "split"): (67.27 + 54.65) * 1e6,
-    ("tile_partition", "fp64"): (29.43 + 35.93) * 1e6,
+    ("propagate", "fp64"): (71.49 + 54.53) * 1e6,
+    ("propagate", "split"): (67.30 + 54.53) * 1e6,
+    ("tile_partition", "fp64"): (29.44 + 34.61) * 1e6,
     ("tile_partition", "split"): (29.45 + 17.83) * 1e6,
-    ("pair_tiles", "fp64"): (56.35 + 0.06) * 1e6,
-    ("pair_tiles", "split"): (32.00 + 0.06) * 1e6,
+    ("pair_tiles", "fp64"): (52.47 + 0.03) * 1e6,
+    ("pair_tiles", "split"): (27.29 + 0.03) * 1e6,
 }
 
 

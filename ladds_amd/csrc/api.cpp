@@ -330,8 +330,8 @@ hipError_t alloc_objects(DeviceObjects &o, size_t cap) {
 constexpr size_t kCrowdingSample = 4096;
 // From this many on the sorting kernel with scan_crowded takes over from the sparse one, which
 // lists every pair before it tests any (clustered populations, one screening, split / FP64,
-// sparse against crowded: 131,072 objects with 9.5 conjunctions each 297 / 360 against 248 / 258
-// us, 524,288 with 40 each in FP64 4020 against 859).
+// sparse against crowded: 131,072 objects with 9.5 conjunctions each 297 / 360 against 193 / 184
+// us, 524,288 with 40 each in FP64 4020 against 580).
 constexpr double kCrowded = 2.0;
 // Four times the buckets per plane: clusters then seldom share one by folding (1,048,576
 // clustered objects, split: 1.70 ms, with twice as many again 2.46).
@@ -553,7 +553,7 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
                         ? (uint32_t)bs
                         : (tp.nscen > 1 ? 128u : (ctx->form == kFormFp64 ? 1024u : 256u));
   if (crowded && !valid_pair_threads(bs)) {
-    // by how full the planes are, 256 / 512 / 1024 threads, us: 64 objects per plane, split
+    // by how full the planes are, 256 / 512 / 1024 threads (us, the fields not yet packed): 64 objects per plane, split
     // 459 / 473 / 617; 256 per plane, split 1972 / 1696 / 2076, FP64 3003 / 2401 / 2144; 128 per
     // plane, FP64 904 / 859 / 1133
     const size_t mean = n / ((size_t)tp.nplanes * tp.nscen);
@@ -657,7 +657,8 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   // scratch arena for planes beyond the LDS capacity: every chunk of a plane sorts it
   tp.crowded = crowded ? 1u : 0u;
   const size_t arena_need = std::max<size_t>(2 * n, 1024) * tp.nchunk;
-  const size_t arena_bytes = arena_need * kArenaSlotBytes;
+  const size_t packed_bytes = crowded ? n * kPackedObjectBytes : 0;  // behind the slots
+  const size_t arena_bytes = arena_need * kArenaSlotBytes + packed_bytes;
   if (tiles && arena_bytes > ctx->scratch_bytes) {
     hipFree(ctx->scratch);
     ctx->scratch = nullptr;
@@ -665,7 +666,8 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     HIPCHK(ctx, hipMalloc(&ctx->scratch, arena_bytes));
     ctx->scratch_bytes = arena_bytes;
   }
-  tp.arena_cap = (uint32_t)std::min<size_t>(ctx->scratch_bytes / kArenaSlotBytes, 0xFFFFFFFFu);
+  const size_t slot_bytes = ctx->scratch_bytes - std::min(ctx->scratch_bytes, packed_bytes);
+  tp.arena_cap = (uint32_t)std::min<size_t>(slot_bytes / kArenaSlotBytes, 0xFFFFFFFFu);
   ctx->tiles = tp;
   const size_t tps_need = (size_t)tp.ntiles * (tp.nplanes + 1);
   if (tps_need > ctx->tps_alloc) {
@@ -1847,7 +1849,7 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
   const double base_cell = 1.0 / ctx->grid.inv_cell;
   const bool ensemble = ctx->tiles.nscen > 1;
   // current point of the search: {plane bits (-1: sized from the objects per plane), threads,
-  // tile, chunks, workgroups per CU, dispatch order, ensemble objects per plane (0: 64), row
+  // tile, chunks, workgroups per CU, dispatch order, ensemble objects per plane (0: 256), row
   // height and bucket width in cells, persistent pair kernel, pair-scan streams (0: by form)}
   double cur_cell = base_cell, cur_fx = 1.0;
   int cur[11] = {-1, (int)ctx->tiles.pair_threads, std::max(4096, (int)ctx->tiles.tile_size),

@@ -66,6 +66,8 @@ constexpr uint32_t kPartitionTile = 8192;
 // Global scratch arena of the pair scan: per record slot a sorted record (32 bytes
 // reserved, the FP64 record's size).
 constexpr size_t kArenaSlotBytes = 32;
+// Behind the slots where cells are crowded: each object's packed predicate fields.
+constexpr size_t kPackedObjectBytes = 80;
 
 // Search radius of the pair scan: the cutoff in the FP64 form; in the split form the
 // FP32 prefilter radius, inflated so that FP32 rounding of positions (< 2^-24 |x| per

@@ -47,41 +47,38 @@ struct SoAObject {
   __device__ __forceinline__ double vz() const { return o.vz[i]; }
 };
 
-// One object's fields in registers: read from the object arrays (`load`), or through the scalar
-// cache when the index is the same for the whole wavefront (`load_uniform`; the kernels that
-// use it do not write the object arrays).
+// What the predicate reads of one object, side by side (k_pack_objects): one or two lines of the
+// cache where the object arrays take eleven.
+struct alignas(16) PackedObject {
+  double r[3], v[3];
+  double rad;
+  uint64_t par, ident;
+  int32_t act;
+  uint32_t pad;
+};
+
+// One object's fields in registers: read from its packed fields, through the scalar cache when the
+// index is the same for the whole wavefront (`load_uniform`; the launch that reads them does
+// not write them).
 struct HeldObject {
   int act;
   uint64_t par, ident;
   double rad, r[3], v[3];
-  __device__ __forceinline__ void load(const DeviceObjects &o, uint32_t i) {
-    act = o.activity[i];
-    rad = o.radius_m[i];
-    par = o.parent[i];
-    ident = o.id[i];
-    r[0] = o.rx[i];
-    r[1] = o.ry[i];
-    r[2] = o.rz[i];
-    v[0] = o.vx[i];
-    v[1] = o.vy[i];
-    v[2] = o.vz[i];
+  template <typename P>
+  __device__ __forceinline__ void from(P *p) {
+    act = p->act;
+    rad = p->rad;
+    par = p->par;
+    ident = p->ident;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      r[k] = p->r[k];
+      v[k] = p->v[k];
+    }
   }
-  template <typename T>
-  static __device__ __forceinline__ T scalar(const T *p, uint32_t i) {
-    typedef const __attribute__((address_space(4))) T *Constant;
-    return ((Constant)(uintptr_t)p)[i];
-  }
-  __device__ __forceinline__ void load_uniform(const DeviceObjects &o, uint32_t i) {
-    act = scalar(o.activity, i);
-    rad = scalar(o.radius_m, i);
-    par = scalar(o.parent, i);
-    ident = scalar(o.id, i);
-    r[0] = scalar(o.rx, i);
-    r[1] = scalar(o.ry, i);
-    r[2] = scalar(o.rz, i);
-    v[0] = scalar(o.vx, i);
-    v[1] = scalar(o.vy, i);
-    v[2] = scalar(o.vz, i);
+  __device__ __forceinline__ void load(const PackedObject *p, uint32_t i) { from(p + i); }
+  __device__ __forceinline__ void load_uniform(const PackedObject *p, uint32_t i) {
+    from((const __attribute__((address_space(4))) PackedObject *)(uintptr_t)(p + i));
   }
   __device__ __forceinline__ int activity() const { return act; }
   __device__ __forceinline__ double radius() const { return rad; }

@@ -333,23 +333,51 @@ __device__ __forceinline__ void scan_plane(const PairTileArgs &a, const RecOf<FO
   }
 }
 
+// The packed fields stand behind the arena's slots.
+__host__ __device__ __forceinline__ PackedObject *packed_objects(void *scratch, const TileParams &tp) {
+  return reinterpret_cast<PackedObject *>(static_cast<char *>(scratch) + (size_t)tp.arena_cap * kArenaSlotBytes);
+}
+
+// 168 bytes an object read and written once, for scan_crowded's reads.
+__global__ __launch_bounds__(256) void k_pack_objects(DeviceObjects o, PackedObject *out) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= o.n) return;
+  PackedObject p;
+  p.r[0] = o.rx[i];
+  p.r[1] = o.ry[i];
+  p.r[2] = o.rz[i];
+  p.v[0] = o.vx[i];
+  p.v[1] = o.vy[i];
+  p.v[2] = o.vz[i];
+  p.rad = o.radius_m[i];
+  p.par = o.parent[i];
+  p.ident = o.id[i];
+  p.act = o.activity[i];
+  p.pad = 0;
+  out[i] = p;
+}
+
 // scan_plane for crowded planes: clusters put tens to thousands of records into one cell, all
 // within R of each other, and nearly every record met is a candidate.  A wavefront takes 64
 // consecutive sorted records, and where their runs in a row nearly coincide (one bucket, or a few
 // neighbours) it walks the union of the runs together: the other record, and its predicate
 // fields read through the scalar cache one ahead, are the same for all lanes, and the own
 // fields stay in registers.  Walked lane by lane, every lane met another record and gathered
-// its fields from eleven arrays (or an 80-byte copy), which bounded the scan.  Runs that do not
-// coincide are walked lane by lane as in scan_plane.  Now bounded by the predicate's FP64
-// instructions in half-filled wavefronts and the fullest planes.  One screening of clustered
-// objects, lane by lane -> here: 1,048,576 with 42 million conjunctions, split 6.38 -> 1.70 ms,
-// FP64 11.2 -> 2.14; 131,072 with 0.62 million, split 0.28 -> 0.25, FP64 0.48 -> 0.26.
+// its fields from eleven arrays (or an 80-byte copy), which bounded the scan.  The fields stand
+// packed by object (k_pack_objects): from the eleven arrays the walk waited for as many lines of
+// the cache a record (1,048,576 clustered objects, split, 1.70 ms, packed 1.16 with the packing;
+// 8,388,608, tuned, 62 and 38 ms per step).  Runs that do not coincide are walked lane by lane
+// as in scan_plane.  Now bounded by the predicate's FP64 instructions in half-filled
+// wavefronts and the fullest planes.  One screening of clustered objects, before -> here:
+// 1,048,576 with 42 million conjunctions, split 6.38 -> 1.16 ms, FP64 11.2 -> 1.47; 131,072
+// with 0.62 million, split 0.28 -> 0.19, FP64 0.48 -> 0.18.
 template <int FORM, bool DIGEST>
 __device__ __forceinline__ void scan_crowded(const PairTileArgs &a, const RecOf<FORM> *sorted,
                                              const uint32_t *cur_own, const uint32_t *cur_halo, uint32_t n_own,
                                              uint32_t threads, uint32_t scen, uint32_t chunk, uint32_t nchunk,
                                              ScanAcc &acc) {
   const GridParams &g = a.g;
+  const PackedObject *packed = packed_objects(a.scratch, a.tp);
   const uint32_t my = (1u << g.by) - 1u, mz = (1u << g.bz) - 1u;
   const uint32_t sy = g.bz, lane = lane_id();
   const bool half = a.tp.half_rows != 0u;
@@ -366,7 +394,7 @@ __device__ __forceinline__ void scan_crowded(const PairTileArgs &a, const RecOf<
     const bool on = s < n_own && (nchunk == 1u || lb % nchunk == chunk);
     if (!__ballot(on)) continue;
     HeldObject mine;
-    mine.load(a.sink.o, me.idx);
+    mine.load(packed, me.idx);
     uint32_t zlo, zhi;
     bool wraps;
     if (a.tp.half_buckets == 0u) {
@@ -415,13 +443,13 @@ __device__ __forceinline__ void scan_crowded(const PairTileArgs &a, const RecOf<
           RecOf<FORM> o = sorted[first];
           uint32_t oj = __builtin_amdgcn_readfirstlane(o.idx);
           HeldObject other;
-          other.load_uniform(a.sink.o, oj);
+          other.load_uniform(packed, oj);
 #pragma unroll 1
           for (uint32_t u = first; u < last; ++u) {
             const RecOf<FORM> p = sorted[min(u + 1u, last - 1u)];
             const uint32_t nj = __builtin_amdgcn_readfirstlane(p.idx);
             HeldObject following;
-            following.load_uniform(a.sink.o, nj);
+            following.load_uniform(packed, nj);
             const bool c = any && u >= q && u < end && within<FORM>(me, o, a.sink.fp);
             if (c) handle_candidate<DIGEST>(a.sink, mine, other, me.idx, oj, acc, scen);
             o = p;
@@ -434,7 +462,7 @@ __device__ __forceinline__ void scan_crowded(const PairTileArgs &a, const RecOf<
             const RecOf<FORM> o = sorted[q];
             if (within<FORM>(me, o, a.sink.fp)) {
               HeldObject other;
-              other.load(a.sink.o, o.idx);
+              other.load(packed, o.idx);
               handle_candidate<DIGEST>(a.sink, mine, other, me.idx, o.idx, acc, scen);
             }
           }
@@ -629,6 +657,7 @@ __device__ __forceinline__ uint32_t xcd_local_item(uint32_t b, uint32_t g) {
 template <int FORM, int THREADS, bool CROWDED>
 constexpr int kPairWavesPerEu = (!CROWDED && (FORM == kFormSplit || THREADS >= 512)) ? 5 : 1;
 
+static_assert(sizeof(PackedObject) == kPackedObjectBytes, "room behind the arena");
 static_assert(sizeof(RecordF64) <= kArenaSlotBytes && sizeof(RecordF32) <= kArenaSlotBytes, "arena slot");
 
 // PERSIST false: one workgroup per plane pair (grid nplanes * nscen * nchunk).
@@ -1205,6 +1234,9 @@ hipError_t launch_pair_tiles(int form, bool digest, const DeviceObjects &o, cons
   if (tp.sparse_threads == 256 && tp.sparse_group == 1) return launch_pair_sparse_as<256, 1>(form, digest, a, s);
   if (tp.sparse_threads == 256 && tp.sparse_group == 2) return launch_pair_sparse_as<256, 2>(form, digest, a, s);
   if (tp.sparse_threads == 512) return launch_pair_sparse_as<512, 1>(form, digest, a, s);
+  if (tp.crowded)
+    hipLaunchKernelGGL(k_pack_objects, dim3((unsigned)((o.n + 255) / 256)), dim3(256), 0, s, o,
+                       packed_objects(scratch, tp));
   switch (tp.pair_threads) {
     case 128:
       launch_pair_tiles_as<128>(form, digest, a, s);

@@ -531,20 +531,34 @@ __global__ __launch_bounds__(kAdjLanes) void k_adjoint_chain(AdjointArgs a) {
   double gbc = (!first && a.g_bc) ? a.g_bc[i] : 0.0;
   // dummies: no gradient flows through a deleted object
   const bool moving = !a.activity || a.activity[i] >= 0;
-#pragma unroll 2
-  for (int c = a.nchunk - 1; c >= 0 && moving; --c) {
-    const double *m = a.phi + (size_t)c * kPhi * n + i;
-    double v[kPhi];
+  // Three matrices in registers: two are on their way while one is applied (a wavefront per CU, so
+  // nothing else hides their reads; 4,096 objects, 45 chunks: 207 -> 24 us).
+  double v[3][kPhi];
+  auto load = [&](double (&m)[kPhi], int c) {
+    const double *p = a.phi + (size_t)c * kPhi * n + i;
 #pragma unroll
-    for (int q = 0; q < kPhi; ++q) v[q] = m[(size_t)q * n];
-    double h[7];
+    for (int q = 0; q < kPhi; ++q) m[q] = p[(size_t)q * n];
+  };
+  const int last = moving ? a.nchunk - 1 : -1;
+  if (last >= 0) load(v[0], last);
+  if (last >= 1) load(v[1], last - 1);
+#pragma unroll 1
+  for (int c0 = last; c0 >= 0; c0 -= 3) {
 #pragma unroll
-    for (int k = 0; k < 7; ++k)
-      h[k] = ((v[6 * k] * g[0] + v[6 * k + 1] * g[1]) + v[6 * k + 2] * g[2]) +
-             ((v[6 * k + 3] * g[3] + v[6 * k + 4] * g[4]) + v[6 * k + 5] * g[5]);
+    for (int k = 0; k < 3; ++k) {
+      const int c = c0 - k;
+      if (c < 0) break;
+      if (c >= 2) load(v[(k + 2) % 3], c - 2);
+      const double (&m)[kPhi] = v[k];
+      double h[7];
 #pragma unroll
-    for (int q = 0; q < 6; ++q) g[q] = h[q];
-    gbc += h[6];
+      for (int j = 0; j < 7; ++j)
+        h[j] = ((m[6 * j] * g[0] + m[6 * j + 1] * g[1]) + m[6 * j + 2] * g[2]) +
+               ((m[6 * j + 3] * g[3] + m[6 * j + 4] * g[4]) + m[6 * j + 5] * g[5]);
+#pragma unroll
+      for (int q = 0; q < 6; ++q) g[q] = h[q];
+      gbc += h[6];
+    }
   }
 #pragma unroll
   for (int q = 0; q < 3; ++q) {

@@ -575,7 +575,8 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   tp.nchunk = (uint32_t)std::min<size_t>(16, std::max<size_t>(1, own_max / (4 * (size_t)tp.pair_threads)));
   // crowded: every chunk sorts the plane again and leaves lanes of the walk idle, so only planes
   // beyond a CU's share of the objects are divided
-  if (crowded) tp.nchunk = (uint32_t)std::max<size_t>(1, std::min<size_t>(tp.nchunk, own_max * 256 / n));
+  if (crowded)
+    tp.nchunk = (uint32_t)std::max<size_t>(1, std::min<size_t>(tp.nchunk, own_max * 256 / std::max<size_t>(n, 1)));
   if (ctx->cfg.scan_chunks >= 1 && ctx->cfg.scan_chunks <= 32) tp.nchunk = (uint32_t)ctx->cfg.scan_chunks;
   if (ctx->tune_chunks >= 1 && ctx->tune_chunks <= 32) tp.nchunk = (uint32_t)ctx->tune_chunks;
   // LDS of a plane pair: room for the fullest plane pair now, then grown to the whole LDS
@@ -1190,7 +1191,9 @@ int compact_if_needed(ladds_ctx *ctx, double burn_r2 = 0.0) {
       const int settled = settle(ctx);
       if (settled != LADDS_OK) return settled;
       if (alive) HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * alive, hipMemcpyDeviceToHost));
-      const int rc = setup_grid(ctx, alive, rx.data());
+      // the shape follows what is left (also nothing), not the population that was measured last
+      int rc = measure_crowding(ctx);
+      if (rc == LADDS_OK) rc = setup_grid(ctx, alive, rx.data());
       if (rc != LADDS_OK) return rc;
     }
   }

@@ -123,7 +123,7 @@ __device__ __forceinline__ void partial_field(double x, double y, double z, unsi
                                               double (&a)[3], Jacobian &o) {
 #pragma clang fp contract(on)
   const double r2 = x * x + y * y + z * z;
-  const double inv_r = rsqrt64(r2);
+  const double inv_r = rsqrt64<true>(r2);
   const double inv_r2 = inv_r * inv_r;
   const double inv_r3 = inv_r2 * inv_r;
   const double inv_r5 = inv_r3 * inv_r2;
@@ -199,10 +199,10 @@ __device__ __forceinline__ void partial_drag(double x, double y, double z, doubl
   const double om = kOmegaEarth;
   const double wx = vx + om * y, wy = vy - om * x, wz = vz;
   const double w2 = wx * wx + wy * wy + wz * wz;
-  const double inv_w = rsqrt64(fmax(w2, 1e-290));
+  const double inv_w = rsqrt64<false>(fmax(w2, 1e-290));
   const double wn = w2 * inv_w;  // 0 without wind
   const double r2 = x * x + y * y + z * z;
-  const double inv_r = rsqrt64(r2);
+  const double inv_r = rsqrt64<true>(r2);
   const double h = r2 * inv_r - kREarth;
   const AtmRow &row = atm_row(h, atm);
   const double inv_scale = row.inv_scale;
@@ -246,7 +246,7 @@ __device__ __forceinline__ void partial_central(double x, double y, double z, co
                                                 const double *indirect, bool gravity, double (&a)[3], Jacobian &o) {
 #pragma clang fp contract(on)
   const double dx = s[0] - x, dy = s[1] - y, dz = s[2] - z;
-  const double inv_d = rsqrt64(dx * dx + dy * dy + dz * dz);
+  const double inv_d = rsqrt64<true>(dx * dx + dy * dy + dz * dz);
   const double inv_d2 = inv_d * inv_d;
   const double f = k * (inv_d2 * inv_d);
   const double go = gravity ? 1.0 : 0.0;

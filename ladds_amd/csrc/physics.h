@@ -72,13 +72,22 @@ inline void fill_atm_table(AtmTable &t) {
   }
 }
 
-// 1/sqrt(x) of a positive normal x: the hardware's estimate (~2^-24) and one cubic step,
-// y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2, which leaves rounding error only.
+// 1/sqrt(x) of a positive x: the hardware's estimate (~2^-24) and one step of third order
+// (Householder's iteration), y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2, which leaves rounding
+// error only.  FAR: x may have overflowed and then gives 0 (its estimate; e is formed with a
+// finite x).  That is one instruction more: paid by every object it took 2% of 1,000 steps of
+// 250,007, so the propagation's paths for the usual models go without and leave the objects
+// beyond kFar to the general one.
+template <bool FAR>
 __device__ __forceinline__ double rsqrt64(double x) {
   const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
+  const double e = fma(-(FAR ? fmin(x, 1.7976931348623157e308) : x) * y, y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
+
+// An object whose coordinates [km] sum up to less at the start of a launch does not come near the
+// overflow of its squared distances within it.
+constexpr double kFar = 1.0e140;
 
 // a b + c with c a constant of the loop.  Written out because the compiler picks the two-address
 // form here and copies the constant into its destination first, one more instruction each.
@@ -171,10 +180,11 @@ constexpr int kEnvWords32 = 3 * (int)sizeof(SubstepEnv<float>) / 8;   // 30
 static_assert(kEnvWords64 <= 64 && kEnvWords32 <= 64, "one word per lane");
 
 // FP64 third body, direct form GM d/|d|^3 - GM s/|s|^3 with d = s - r; returns 1/|d|^3.
+template <bool FAR>
 __device__ __forceinline__ double third_body64(double dx, double dy, double dz, double gm, const double *acc,
                                                bool gravity, double &ax, double &ay, double &az) {
 #pragma clang fp contract(off)
-  const double inv_d = rsqrt64(fma(dz, dz, fma(dx, dx, dy * dy)));
+  const double inv_d = rsqrt64<FAR>(fma(dz, dz, fma(dx, dx, dy * dy)));
   const double inv_d3 = inv_d * inv_d * inv_d;
   if (gravity) {
     const double f = gm * inv_d3;
@@ -223,7 +233,7 @@ __device__ __forceinline__ void drag_term64(double x, double y, double vx, doubl
   const double om = kOmegaEarth;
   const double wx = fma(om, y, vx), wy = fma(-om, x, vy), wz = vz;
   const double w2 = fma(wz, wz, fma(wx, wx, wy * wy));
-  const double vn = w2 * rsqrt64(fmax(w2, 1e-290));  // 0 without wind
+  const double vn = w2 * rsqrt64<false>(fmax(w2, 1e-290));  // 0 without wind
   const double f = drag64 * atm_density(h, t) * vn;
   ax = fma(f, wx, ax);
   ay = fma(f, wy, ay);
@@ -244,15 +254,15 @@ struct ObjParams {
 // rounds alike, and the components are added one after the other, Kepler first.  Merged into
 // one factor on the position they would cost ~10 instructions fewer, but a differently rounded
 // Kepler or J2 term shows in a pair's squared distance after some hundred steps (3e-9
-// relative after four hours).  SRP shares the Sun's geometry.
-template <int FORM>
+// relative after four hours).  SRP shares the Sun's geometry.  FAR: see rsqrt64.
+template <int FORM, bool FAR>
 __device__ __forceinline__ void acceleration(double x, double y, double z, double vx, double vy, double vz,
                                              const ObjParams &p, unsigned mask, const SubstepEnv<double> &e64,
                                              const SubstepEnv<float> &e32, const AtmTable &atm, double &ax,
                                              double &ay, double &az) {
 #pragma clang fp contract(off)
   const double r2 = fma(z, z, fma(x, x, y * y));
-  const double inv_r = rsqrt64(r2);
+  const double inv_r = rsqrt64<FAR>(r2);
   const double inv_r2 = inv_r * inv_r;
   const double inv_r3 = inv_r2 * inv_r;
   // (chosen, not multiplied by 0: without this force an object at the origin, or infinitely far, has none)
@@ -285,11 +295,11 @@ __device__ __forceinline__ void acceleration(double x, double y, double z, doubl
       dx = e64.sun[0] - x;
       dy = e64.sun[1] - y;
       dz = e64.sun[2] - z;
-      const double inv_d3 = third_body64(dx, dy, dz, kGmSun, e64.sun_acc, (mask & kSolBit) != 0, ax, ay, az);
+      const double inv_d3 = third_body64<FAR>(dx, dy, dz, kGmSun, e64.sun_acc, (mask & kSolBit) != 0, ax, ay, az);
       if (mask & kSrpBit) srp = (in_shadow(x, y, z, r2, e64) ? 0.0 : -p.srp64) * inv_d3;
     }
     if (mask & kLunBit)
-      third_body64(e64.moon[0] - x, e64.moon[1] - y, e64.moon[2] - z, kGmMoon, e64.moon_acc, true, ax, ay, az);
+      third_body64<FAR>(e64.moon[0] - x, e64.moon[1] - y, e64.moon[2] - z, kGmMoon, e64.moon_acc, true, ax, ay, az);
     if (mask & kSrpBit) {  // srp (r - s)/|r - s|^3
       ax = fma(srp, dx, ax);
       ay = fma(srp, dy, ay);

@@ -15,6 +15,8 @@
 // Several steps per launch keep the state in registers between steps (used when
 // no conjunction scan is due in between).  When `count` is set, the kernel also
 // performs the counting pass of the cell binning for the final positions.
+#include <type_traits>
+
 #include "binning.h"
 #include "launch.h"
 #include "physics.h"
@@ -139,18 +141,20 @@ __global__ __launch_bounds__(256) void k_propagate(PropagateArgs a) {
   };
   // The two usual models, without evasivePreserving objects in the wavefront, with a constant
   // mask: one block of straight code per kick, whose components' chains interleave (4,099
-  // objects, full model, FP64: 2.05 -> 1.62 us per step; 1,048,576: 22.9 -> 20.3 us).
-  auto with = [&](unsigned m) {
+  // objects, full model, FP64: 2.05 -> 1.62 us per step; 1,048,576: 22.9 -> 20.3 us).  The path of all
+  // others also takes objects beyond kFar (or not numbers).
+  auto with = [&](unsigned m, auto far) {
     return [&, m](const SubstepEnv<double> &e64, const SubstepEnv<float> &e32, double &ax, double &ay, double &az) {
-      acceleration<FORM>(x, y, z, vx, vy, vz, p, m, e64, e32, atm, ax, ay, az);
+      acceleration<FORM, decltype(far)::value>(x, y, z, vx, vy, vz, p, m, e64, e32, atm, ax, ay, az);
     };
   };
-  if (__ballot(mask != kAllBits) == 0ull)
-    steps(with(kAllBits));
-  else if (__ballot(mask != (kKepBit | kJ2Bit)) == 0ull)
-    steps(with(kKepBit | kJ2Bit));
+  const bool far = !(fabs(x) + fabs(y) + fabs(z) < kFar);
+  if (__ballot(mask != kAllBits || far) == 0ull)
+    steps(with(kAllBits, std::false_type{}));
+  else if (__ballot(mask != (kKepBit | kJ2Bit) || far) == 0ull)
+    steps(with(kKepBit | kJ2Bit, std::false_type{}));
   else
-    steps(with(mask));
+    steps(with(mask, std::true_type{}));
   if (!live) return;
   if (burnt) {
     a.oact[i] = -1;

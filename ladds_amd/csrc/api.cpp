@@ -163,7 +163,14 @@ struct ladds_ctx {
   uint32_t *d_plane_order = nullptr;
   size_t plane_order_alloc = 0;
 
-  double crowding = 0.0;  // objects in an object's own cell, from a sample (crowding_of)
+  // Objects that share cells, as measure_crowding counted them: the mean number of others in an
+  // object's cell and the most in one cell.  Since then (follow_cells): detections, and the fewest
+  // candidates of one (< 0: none yet).
+  double crowding = 0.0;
+  uint32_t fullest_cell = 0;
+  uint64_t detections = 0;
+  double candidates = -1.0;
+  bool tuning = false;  // ladds_autotune times shapes: none is changed beside it
 
   // Autotuned plane-tile shape (ladds_autotune); zero / negative values keep the defaults.
   double tune_cell_km = 0.0;
@@ -324,52 +331,44 @@ hipError_t alloc_objects(DeviceObjects &o, size_t cap) {
   return e;
 }
 
-// Mean number of other objects in an object's cell (side `cell`, same scenario), estimated from
-// a sample of at most kCrowdingSample objects spread over the indices; position(i, p) gives
-// the position of object i.  Populations in low orbits have ~1e-3; clusters have their size.
-constexpr size_t kCrowdingSample = 4096;
-// From this many on the sorting kernel with scan_crowded takes over from the sparse one, which
-// lists every pair before it tests any (clustered populations, one screening, split / FP64,
-// sparse against crowded: 131,072 objects with 9.5 conjunctions each 297 / 360 against 193 / 184
-// us, 524,288 with 40 each in FP64 4020 against 580).
-constexpr double kCrowded = 2.0;
+// Which pair kernel suits the objects, by how they share cells (measure_crowding).  The sparse kernel
+// lists every pair of a cell before it tests any, in one workgroup: a lone cloud of k costs it ~12 ns
+// for each of its k^2 ordered pairs.
+//   crowded  the sorting kernel with scan_crowded, from a mean of kCrowded others in an object's cell on
+//            (clustered populations, one screening, split / FP64, sparse against crowded: 131,072
+//            objects with 9.5 conjunctions each 297 / 360 against 193 / 184 us, 524,288 with 40 each
+//            in FP64 4020 against 580), and where clouds alone make a mean of kCrowdedClouds
+//   clouds   the sorting kernel in the shape of a sparse population, from kCloud objects in one cell on
+// A cloud of k fragments among n, one detection / a step of ladds_simulate, us, sparse against clouds
+// against crowded.  n 1,048,576, split: k 60 122 / 58, 130 / 69, 160 / 148; k 100 209 / 64, 161 / 77, 184
+// / 155; k 150 368 / 80, 204 / 86, 235 / 160; k 1000 11622 / 1487, 2771 / 493, 1267 / 408; FP64: k 100 223
+// / 94, 214 / 157, 202 / 224; k 150 362 / 129, 258 / 168, 236 / 240; k 300 1273 / 340, 397 / 223, 338 /
+// 302.  n 65,521, split: k 100 236 / 36, 136 / 42, 112 / 44; k 600 6119 / 652, 1171 / 231, 769 / 201.
+constexpr double kCrowded = 2.0, kCrowdedClouds = 0.5;
+constexpr uint32_t kCloud64 = 128, kCloudSplit = 96;
+enum CellShape { kSparseCells, kCloudCells, kCrowdedCells };
+
+CellShape cell_shape(const ladds_ctx *ctx) {
+  const bool cloud = ctx->fullest_cell >= (ctx->form == kFormFp64 ? kCloud64 : kCloudSplit);
+  if (ctx->crowding >= kCrowded || (cloud && ctx->crowding >= kCrowdedClouds)) return kCrowdedCells;
+  return cloud ? kCloudCells : kSparseCells;
+}
+
 // Four times the buckets per plane: clusters then seldom share one by folding (1,048,576
 // clustered objects, split: 1.70 ms, with twice as many again 2.46).
 constexpr uint32_t kCrowdedBits = 2;
 
-size_t crowding_index(size_t k, size_t m, size_t n) {
-  uint64_t h = (k + 1) * 0x9E3779B97F4A7C15ull;  // a place of its own in the k-th of m equal parts
-  h ^= h >> 32;
-  const size_t lo = k * n / m, hi = (k + 1) * n / m;
-  return lo + (size_t)(h % std::max<size_t>(1, hi - lo));
-}
-
-template <typename F>
-double crowding_of(size_t n, const std::vector<uint64_t> &scen_off, double cell, F &&position) {
-  const size_t m = std::min(n, kCrowdingSample);
-  if (m < 2) return 0.0;
-  std::vector<uint64_t> key(m);
-  size_t scen = 0;
-  for (size_t k = 0; k < m; ++k) {
-    const size_t i = crowding_index(k, m, n);
-    while (scen + 2 < scen_off.size() && i >= scen_off[scen + 1]) ++scen;
-    double p[3];
-    position(k, i, p);
-    uint64_t h = scen;
-    for (int c = 0; c < 3; ++c) {
-      const double u = std::fmin(std::fmax(p[c] / cell, -1.0e9), 1.0e9);
-      h = (h ^ (uint64_t)(int64_t)std::floor(u)) * 0x9E3779B97F4A7C15ull;
-      h ^= h >> 29;
-    }
-    key[k] = h;
-  }
-  std::sort(key.begin(), key.end());
-  double pairs = 0.0;
-  for (size_t k = 0, run = 0; k < m; ++k) {
-    run = (k && key[k] == key[k - 1]) ? run + 1 : 0;
-    pairs += (double)run;
-  }
-  return 2.0 * pairs / (double)m * (double)(n - 1) / (double)(m - 1);
+// Side of the cells along y and z [km].
+int cell_side(ladds_ctx *ctx, double *cell) {
+  const bool tiles = ctx->variant == kVariantPlaneTiles;
+  const double min_cell = (tiles ? 1.0 : 2.0) * search_radius(ctx->form, ctx->cfg.cutoff_km) * (1.0 + 1e-9);
+  *cell = ctx->cfg.cell_size_km > 0.0 ? ctx->cfg.cell_size_km : min_cell;
+  if (tiles && ctx->tune_cell_km > 0.0) *cell = ctx->tune_cell_km;
+  if (!(*cell >= min_cell))
+    return ctx->fail(LADDS_E_INVALID, tiles ? "cell_size_km must be >= the search radius (cutoff, or the split "
+                                              "prefilter radius)"
+                                            : "cell_size_km must be >= 2 * the search radius");
+  return LADDS_OK;
 }
 
 // Grid geometry.  Atomic counting sort: cells of side >= 2R, 2x2x2 search blocks, about
@@ -379,14 +378,9 @@ double crowding_of(size_t n, const std::vector<uint64_t> &scen_off, double cell,
 int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   ctx->keys_valid = false;
   const bool tiles = ctx->variant == kVariantPlaneTiles;
-  const double radius = search_radius(ctx->form, ctx->cfg.cutoff_km);
-  const double min_cell = (tiles ? 1.0 : 2.0) * radius * (1.0 + 1e-9);
-  double cell = ctx->cfg.cell_size_km > 0.0 ? ctx->cfg.cell_size_km : min_cell;
-  if (tiles && ctx->tune_cell_km > 0.0) cell = ctx->tune_cell_km;
-  if (!(cell >= min_cell))
-    return ctx->fail(LADDS_E_INVALID, tiles ? "cell_size_km must be >= the search radius (cutoff, or the split "
-                                              "prefilter radius)"
-                                            : "cell_size_km must be >= 2 * the search radius");
+  double cell = 0.0;
+  const int checked = cell_side(ctx, &cell);
+  if (checked != LADDS_OK) return checked;
   GridParams g{};
   g.inv_cell = 1.0 / cell;
   // plane width: cells may be longer in x than in y and z (fewer, fuller planes)
@@ -394,7 +388,7 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   g.inv_cell_x = 1.0 / cell_x;
   // buckets two cells tall (wide): an object then scans two rows of the next plane (two
   // buckets of a row), not three
-  const bool crowded = ctx->crowding >= kCrowded;
+  const bool crowded = cell_shape(ctx) == kCrowdedCells;
   const bool half_rows = tiles && (ctx->tune_rows == 2 || (ctx->tune_rows == 0 && crowded));
   const bool half_buckets = tiles && (ctx->tune_bcells == 2 || (ctx->tune_bcells == 0 && crowded));
   g.inv_cell_y = half_rows ? 0.5 * g.inv_cell : g.inv_cell;
@@ -558,6 +552,12 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     // plane, FP64 904 / 859 / 1133
     const size_t mean = n / ((size_t)tp.nplanes * tp.nscen);
     tp.pair_threads = mean < 96 ? 256u : ((ctx->form == kFormFp64 && mean >= 192) ? 1024u : 512u);
+    // a cloud that makes a quarter of all pairs in cells is one plane's, and its workgroup's time the
+    // scan's: 256 / 512 / 1024 threads, 65,521 objects, FP64, cloud of 300 332 / 279 / 274 us, of 1,000
+    // 1880 / 1141 / 828; 1,048,576, split, of 1,000 - / 1259 / 912
+    const double k = (double)ctx->fullest_cell;
+    if (4.0 * k * k >= ctx->crowding * (double)n && k >= 256.0)
+      tp.pair_threads = std::max(tp.pair_threads, k >= 512.0 ? 1024u : 512u);
   }
   if (valid_pair_threads(ctx->tune_threads)) tp.pair_threads = (uint32_t)ctx->tune_threads;
   tp.lds_header_words = pair_tiles_header_words(tp);  // depends on the workgroup size
@@ -612,7 +612,7 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
     const size_t cap = share > hdr + kLdsMargin ? (share - hdr - kLdsMargin) / rec / 64 * 64 : 0;
     tp.cap_items = (uint32_t)std::min(fit, std::max<size_t>(cap, 256));
   }
-  // Sparse pair kernel, unless cells are crowded, a plane and the next one exceed its LDS, the
+  // Sparse pair kernel, unless cells hold clouds, a plane and the next one exceed its LDS, the
   // configuration or the tuner asked for chunks or persistent workgroups or the configuration names
   // a workgroup size of the sorting kernel.
   // Two planes per workgroup where planes are full and enough for every CU (pair kernel by events:
@@ -624,7 +624,7 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   const bool chunks_chosen = (ctx->cfg.scan_chunks >= 1 && ctx->cfg.scan_chunks <= 32) ||
                              (ctx->tune_chunks >= 1 && ctx->tune_chunks <= 32);
   if (tiles && !plane_count.empty() && !(chunks_chosen && tp.nchunk > 1) && tp.persistent_groups == 0u &&
-      !valid_pair_threads(bs) && !crowded) {
+      !valid_pair_threads(bs) && cell_shape(ctx) == kSparseCells) {
     // most records of a group of planes and the next one, with room for their drift
     auto group_max = [&](size_t group) {
       const size_t P = tp.nplanes;
@@ -750,31 +750,79 @@ int settle(ladds_ctx *ctx) {
     if (settle_rc != LADDS_OK) return settle_rc; \
   } while (0)
 
-// The crowding of the objects on the device (after scenarios or objects changed): the sample's
-// positions are gathered and read back.
-int measure_crowding(ladds_ctx *ctx) {
-  const size_t n = ctx->n, m = std::min(n, kCrowdingSample);
-  ctx->crowding = 0.0;
-  if (m < 2) return LADDS_OK;
-  std::vector<uint32_t> idx(m);
-  std::vector<double> state(6 * m);
-  for (size_t k = 0; k < m; ++k) idx[k] = (uint32_t)crowding_index(k, m, n);
-  char *buf = nullptr;
-  const size_t out = (sizeof(uint32_t) * m + 255) / 256 * 256;
-  HIPCHK(ctx, hipMalloc(reinterpret_cast<void **>(&buf), out + sizeof(double) * 6 * m));
-  double *got = reinterpret_cast<double *>(buf + out);
-  hipError_t e = hipMemcpyAsync(buf, idx.data(), sizeof(uint32_t) * m, hipMemcpyHostToDevice, ctx->stream);
-  if (e == hipSuccess)
-    e = launch_gather_state(ctx->d, reinterpret_cast<const uint32_t *>(buf), m, got, ctx->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(state.data(), got, sizeof(double) * 6 * m, hipMemcpyDeviceToHost, ctx->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-  hipFree(buf);
-  if (e != hipSuccess) return ctx->hipfail(e, "crowding sample");
-  ctx->crowding = crowding_of(n, ctx->scen_off, ctx->cfg.cutoff_km, [&](size_t k, size_t, double *p) {
-    for (int c = 0; c < 3; ++c) p[c] = state[6 * k + c];
-  });
+int ensure_xbuf(ladds_ctx *ctx, size_t bytes) {
+  if (!ctx->xcount) HIPCHK(ctx, dalloc(&ctx->xcount, 2));
+  if (bytes <= ctx->xbuf_bytes) return LADDS_OK;
+  hipFree(ctx->xbuf);
+  ctx->xbuf = nullptr;
+  ctx->xbuf_bytes = 0;
+  HIPCHK(ctx, hipMalloc(&ctx->xbuf, bytes));
+  ctx->xbuf_bytes = bytes;
   return LADDS_OK;
+}
+
+// Counts the objects on the device by cell (side: the search radius; same scenario).  The table
+// takes the place of the records, which every detection writes anew.
+int measure_crowding(ladds_ctx *ctx) {
+  const size_t n = ctx->n;
+  ctx->crowding = 0.0;
+  ctx->fullest_cell = 0;
+  ctx->candidates = -1.0;
+  ctx->detections = 0;
+  if (n < 2 || ctx->variant != kVariantPlaneTiles) return LADDS_OK;
+  const size_t nscen = ctx->scen_off.size() > 2 ? ctx->scen_off.size() - 1 : 1;
+  const size_t off_bytes = nscen > 1 ? sizeof(uint64_t) * (nscen + 1) : 0;
+  if (off_bytes) {
+    const int rc = ensure_xbuf(ctx, off_bytes);
+    if (rc != LADDS_OK) return rc;
+  }
+  // 4n to 8n words, at most the records' 32 bytes an object
+  const size_t words = (size_t)1 << std::min<uint32_t>(32u, ceil_log2(4 * (uint64_t)n));
+  static_assert(sizeof(RecordF64) >= 8 * sizeof(uint32_t), "the table fits the records");
+  if (off_bytes)
+    HIPCHK(ctx, hipMemcpyAsync(ctx->xbuf, ctx->scen_off.data(), off_bytes, hipMemcpyHostToDevice, ctx->stream));
+  HIPCHK(ctx, hipMemsetAsync(ctx->rec, 0, sizeof(uint32_t) * words, ctx->stream));
+  // (the first two counters, which every detection sets to 0 before it counts)
+  unsigned long long *out = reinterpret_cast<unsigned long long *>(ctx->counters);
+  static_assert(offsetof(ScanCounters, hits) == 0 && offsetof(ScanCounters, evaded) == 8, "two words");
+  HIPCHK(ctx, hipMemsetAsync(out, 0, 2 * sizeof(unsigned long long), ctx->stream));
+  const double inv_cell = 1.0 / search_radius(ctx->form, ctx->cfg.cutoff_km);
+  HIPCHK(ctx, launch_cell_crowding(ctx->d, inv_cell, off_bytes ? static_cast<const uint64_t *>(ctx->xbuf) : nullptr,
+                                   (uint32_t)nscen, static_cast<uint32_t *>(ctx->rec), (uint32_t)(words - 1), out,
+                                   ctx->stream));
+  HIPCHK(ctx, launch_publish(out, reinterpret_cast<unsigned long long *>(&ctx->d_rb_host->sc), 2, ctx->stream));
+  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+  const uint64_t pairs = ctx->h_rb->sc.hits, fullest = ctx->h_rb->sc.evaded;
+  const double by_chance = (double)(n - 1) / (double)words;  // cells that share an entry of the table
+  ctx->crowding = std::max(0.0, 2.0 * (double)pairs / (double)n - by_chance);
+  ctx->fullest_cell = (uint32_t)fullest;
+  return LADDS_OK;
+}
+
+// The shape for the objects on the device (the host needs their x coordinates).
+int reshape(ladds_ctx *ctx) {
+  std::vector<double> rx(ctx->n);
+  if (ctx->n) HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * ctx->n, hipMemcpyDeviceToHost));
+  return setup_grid(ctx, ctx->n, rx.data());
+}
+
+// Called after `detections` detections that met `candidates` pairs within the search radius: clouds
+// disperse, and others may form, and the pair scan's shape follows.  Cells are counted again after
+// every kCellsAgain detections of a population with clouds, and for others where a detection meets
+// more than twice as many pairs as before.  (Counting takes ~60 us at 1,000,000 objects.)
+int follow_cells(ladds_ctx *ctx, uint64_t candidates, uint64_t detections) {
+  if (detections == 0 || ctx->n < 2 || ctx->variant != kVariantPlaneTiles || ctx->tuning) return LADDS_OK;
+  constexpr uint64_t kCellsAgain = 64;
+  constexpr double kFew = 2000.0;  // half the pairs of a cell of kCloudSplit
+  const CellShape shape = cell_shape(ctx);
+  const double now = (double)candidates / (double)detections;
+  ctx->detections += detections;
+  ctx->candidates = ctx->candidates < 0.0 ? now : std::min(ctx->candidates, now);
+  if (shape == kSparseCells ? now < 2.0 * ctx->candidates + kFew : ctx->detections < kCellsAgain) return LADDS_OK;
+  int rc = measure_crowding(ctx);
+  ctx->candidates = now;
+  if (rc == LADDS_OK && cell_shape(ctx) != shape) rc = reshape(ctx);
+  return rc;
 }
 
 int ensure_log(ladds_ctx *ctx, uint64_t cap) {
@@ -1104,7 +1152,9 @@ constexpr size_t kSerialGraphObjects = 262144;
 // Up to here the eager loop, too, puts the three kernels of a step on one stream (us per step,
 // serial against overlapped with the partition behind the propagation: 4,096 objects, FP64, 17.8
 // against 20.2; 16,384 19.5 and 22.5; 32,768 21.3, 19 to 23; 65,521 split 22.0, 16 to 20). With a
-// detection in every third step or fewer the streams stay: the other steps are one launch.
+// detection in every third step or fewer the streams stay: the other steps are one launch.  So they
+// do where cells hold clouds, whose scans are long (16,384 objects, a cloud of 400, split: 100 to 120
+// us per step, 210 on one stream).
 constexpr size_t kSerialObjects = 32768;
 
 // Step graph of `steps` steps from state buffer b.  Each step: the pair scan of the state in b,
@@ -1187,13 +1237,10 @@ int compact_if_needed(ladds_ctx *ctx, double burn_r2 = 0.0) {
         off[sc + 1] = off[sc] + kept;
       }
       ctx->scen_off = off;
-      std::vector<double> rx(alive);
-      const int settled = settle(ctx);
-      if (settled != LADDS_OK) return settled;
-      if (alive) HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * alive, hipMemcpyDeviceToHost));
       // the shape follows what is left (also nothing), not the population that was measured last
-      int rc = measure_crowding(ctx);
-      if (rc == LADDS_OK) rc = setup_grid(ctx, alive, rx.data());
+      int rc = settle(ctx);
+      if (rc == LADDS_OK) rc = measure_crowding(ctx);
+      if (rc == LADDS_OK) rc = reshape(ctx);
       if (rc != LADDS_OK) return rc;
     }
   }
@@ -1541,20 +1588,19 @@ int ladds_set_objects(ladds_ctx *ctx, const ladds_objects *o) {
   HIPCHK(ctx, hipSetDevice(ctx->device));
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
   const size_t n = o->n;
-  rc = reserve_objects(ctx, n, false);
+  double cell = 0.0;
+  rc = cell_side(ctx, &cell);
+  if (rc == LADDS_OK) rc = reserve_objects(ctx, n, false);
   if (rc != LADDS_OK) return rc;
   ctx->scen_off.clear();  // a new population is a single scenario until ladds_set_scenarios
-  ctx->crowding = crowding_of(n, ctx->scen_off, ctx->cfg.cutoff_km, [&](size_t, size_t i, double *p) {
-    p[0] = o->rx[i];
-    p[1] = o->ry[i];
-    p[2] = o->rz[i];
-  });
-  rc = setup_grid(ctx, n, o->rx);
-  if (rc != LADDS_OK) return rc;
   ctx->n = n;
   ctx->d.n = n;
   ctx->protected_objects = has_parents(o);
-  return upload_objects(ctx, o, 0);
+  rc = upload_objects(ctx, o, 0);
+  if (rc == LADDS_OK) rc = measure_crowding(ctx);
+  if (rc == LADDS_OK) rc = setup_grid(ctx, n, o->rx);
+  if (rc != LADDS_OK) ctx->n = ctx->d.n = 0;
+  return rc;
 }
 
 int ladds_add_objects(ladds_ctx *ctx, const ladds_objects *o) {
@@ -1575,10 +1621,7 @@ int ladds_add_objects(ladds_ctx *ctx, const ladds_objects *o) {
   ctx->d.n = n;
   ctx->protected_objects = ctx->protected_objects || has_parents(o);
   rc = measure_crowding(ctx);
-  if (rc != LADDS_OK) return rc;
-  std::vector<double> rx(n);
-  HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * n, hipMemcpyDeviceToHost));
-  return setup_grid(ctx, n, rx.data());
+  return rc == LADDS_OK ? reshape(ctx) : rc;
 }
 
 int ladds_set_scenarios(ladds_ctx *ctx, size_t nscenarios, const uint64_t *offsets) {
@@ -1597,10 +1640,7 @@ int ladds_set_scenarios(ladds_ctx *ctx, size_t nscenarios, const uint64_t *offse
   else
     ctx->scen_off.assign(offsets, offsets + nscenarios + 1);
   const int rc = measure_crowding(ctx);
-  if (rc != LADDS_OK) return rc;
-  std::vector<double> rx(ctx->n);
-  HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * ctx->n, hipMemcpyDeviceToHost));
-  return setup_grid(ctx, ctx->n, rx.data());
+  return rc == LADDS_OK ? reshape(ctx) : rc;
 }
 
 size_t ladds_num_scenarios(const ladds_ctx *ctx) {
@@ -1833,6 +1873,11 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
   const size_t n = ctx->n;
   std::vector<double> rx(n);
   HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * n, hipMemcpyDeviceToHost));
+  struct Tuning {  // (a timed burst of steps leaves the shape alone)
+    ladds_ctx *ctx;
+    explicit Tuning(ladds_ctx *c) : ctx(c) { ctx->tuning = true; }
+    ~Tuning() { ctx->tuning = false; }
+  } tuning(ctx);
   // start from the untuned default
   ctx->tune_cell_km = 0.0;
   ctx->tune_pb = -1;
@@ -2027,20 +2072,6 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
 
 }  // extern "C"
 
-namespace {
-
-int ensure_xbuf(ladds_ctx *ctx, size_t bytes) {
-  if (!ctx->xcount) HIPCHK(ctx, dalloc(&ctx->xcount, 2));
-  if (bytes <= ctx->xbuf_bytes) return LADDS_OK;
-  hipFree(ctx->xbuf);
-  ctx->xbuf = nullptr;
-  ctx->xbuf_bytes = 0;
-  HIPCHK(ctx, hipMalloc(&ctx->xbuf, bytes));
-  ctx->xbuf_bytes = bytes;
-  return LADDS_OK;
-}
-
-}  // namespace
 
 extern "C" {
 
@@ -2074,10 +2105,8 @@ int ladds_set_tuning(ladds_ctx *ctx, const ladds_tuning *t) {
   ctx->tune_persistent = t->persistent;
   ctx->tune_pair_streams = t->pair_streams;
   if (ctx->n == 0) return LADDS_OK;  // applied at the next ladds_set_objects
-  std::vector<double> rx(ctx->n);
   HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  HIPCHK(ctx, hipMemcpy(rx.data(), ctx->d.rx, sizeof(double) * ctx->n, hipMemcpyDeviceToHost));
-  return setup_grid(ctx, ctx->n, rx.data());
+  return reshape(ctx);
 }
 
 int ladds_conjunctions(ladds_ctx *ctx, double dt_interp, ladds_pair *hits, size_t cap, size_t *n, ladds_pair *evaded,
@@ -2152,7 +2181,7 @@ int ladds_conjunctions(ladds_ctx *ctx, double dt_interp, ladds_pair *hits, size_
   *n = nh;
   *ne = nev;
   if (nh > cap || nev > ecap) return ctx->fail(LADDS_E_OVERFLOW, "pair output capacity too small");
-  return LADDS_OK;
+  return follow_cells(ctx, ctx->h_rb->sc.candidates, 1);
 }
 
 int ladds_gather_state(ladds_ctx *ctx, const uint32_t *idx, size_t count, double *r, double *v) {
@@ -2215,7 +2244,7 @@ int ladds_conjunction_digest(ladds_ctx *ctx, double dt_interp, uint64_t *n, uint
   digest[1] = sc.digest[1];
   edigest[0] = sc.edigest[0];
   edigest[1] = sc.edigest[1];
-  return LADDS_OK;
+  return follow_cells(ctx, sc.candidates, 1);
 }
 
 int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpcd, double min_altitude_km,
@@ -2238,7 +2267,7 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
   const bool use_graph = ctx->cfg.step_graph != 0 && tpcd == 1 && ctx->variant == kVariantPlaneTiles &&
                          !ctx->profiling && ctx->n > 0 && nsteps > 0;
   const bool use_overlap = !use_graph && ctx->variant == kVariantPlaneTiles && ctx->n > 0 && nsteps > 0 &&
-                           (ctx->n > kSerialObjects || tpcd > 2);
+                           (ctx->n > kSerialObjects || tpcd > 2 || cell_shape(ctx) != kSparseCells);
   // The eager loop's first iteration runs on stream2 (overlapped_iteration's `fill`), and so
   // does what precedes it here (counter reset, spawn state, environments), after anything
   // still queued on the context's stream.
@@ -2258,6 +2287,7 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
   // accounts the iterations since the previous one (span), trailing iterations at the end.
   const bool spawn = ctx->protected_objects && ctx->n > 0 && nsteps > 0;
   uint64_t next_acc = first_iteration;  // first iteration whose start is not accounted yet
+  uint64_t detections = 0;
   if (spawn) {
     if (!ctx->d_spawn) HIPCHK(ctx, dalloc(&ctx->d_spawn, 1));
     ctx->h_rb->spawn = SpawnState{ctx->quiet, 0ull, 0ull, 0ull};
@@ -2339,6 +2369,7 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
         return rc;
       }
       next_acc = base + (uint64_t)seg;
+      detections += (uint64_t)seg;
       ctx->step_count += (uint64_t)seg;
       continue;
     }
@@ -2354,6 +2385,7 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
       const bool detect = (it % (uint64_t)tpcd) == 0;
       const uint64_t span = (spawn && detect) ? it - next_acc + 1 : 0;
       if (detect) next_acc = spawn ? it + 1 : next_acc;
+      detections += detect ? 1 : 0;
       int rc;
       if (use_overlap) {
         const int nxt = (cur + 1) % nbuf;
@@ -2467,7 +2499,7 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
     stats->edigest[1] = sc.edigest[1];
     stats->remaining = ctx->n;
   }
-  return LADDS_OK;
+  return follow_cells(ctx, sc.candidates, detections);
 }
 
 int ladds_remove_spawn_protection(ladds_ctx *ctx) {

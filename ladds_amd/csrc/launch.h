@@ -50,6 +50,11 @@ hipError_t launch_pair_tiles(int form, bool digest, const DeviceObjects &o, cons
                              void *scratch, uint32_t *arena_top, LoggedPair *log, uint64_t log_cap,
                              unsigned long long *log_count, ScanCounters *counters, uint64_t iteration,
                              const StepState *step_state, hipStream_t s);
+// Objects per cell (of the scenario, with scen_off: nscen + 1 offsets on the device): out[0] gets the
+// pairs of objects in one cell, out[1] the fullest cell (0: no cell with two).  `table`: mask + 1
+// zeroed words, out zeroed.
+hipError_t launch_cell_crowding(const DeviceObjects &o, double inv_cell, const uint64_t *scen_off,
+                                uint32_t nscen, uint32_t *table, uint32_t mask, unsigned long long *out, hipStream_t s);
 uint32_t pair_tiles_header_words(const TileParams &tp);
 // LDS bytes of a workgroup of the sparse pair kernel (TileParams::sparse_threads > 0).
 size_t pair_sparse_lds_bytes(const TileParams &tp);

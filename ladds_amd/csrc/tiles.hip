@@ -333,6 +333,52 @@ __device__ __forceinline__ void scan_plane(const PairTileArgs &a, const RecOf<FO
   }
 }
 
+// Objects per cell: every object counts itself into its cell's entry of a hash table (`mask` + 1
+// zeroed words, several for each object) and sees how many were there before it.  out[0]: the sum
+// of those, out[1]: the fullest entry.  Cells that share an entry add to the sum by chance.  Bound
+// by the atomics' way to the caches and back; few wavefronts take many objects each, so that the
+// two totals are not what it waits for.
+__global__ __launch_bounds__(256) void k_cell_crowding(DeviceObjects o, double inv_cell,
+                                                       const uint64_t *scen_off, uint32_t nscen, uint32_t *table,
+                                                       uint32_t mask, unsigned long long *out) {
+  unsigned long long before = 0;
+  uint32_t most = 0;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < o.n; i += (size_t)gridDim.x * 256) {
+    uint32_t lo = 0;
+    if (scen_off) {
+      uint32_t hi = nscen;
+      while (hi - lo > 1u) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (scen_off[mid] <= i)
+          lo = mid;
+        else
+          hi = mid;
+      }
+    }
+    uint32_t low;
+    const uint32_t ix = (uint32_t)cell_axis(o.rx[i], inv_cell, low), iy = (uint32_t)cell_axis(o.ry[i], inv_cell, low),
+                   iz = (uint32_t)cell_axis(o.rz[i], inv_cell, low);
+    const uint64_t h = mix64((((uint64_t)lo << 32) | ix) ^ mix64(((uint64_t)iy << 32) | iz));
+    const uint32_t there = atomicAdd(&table[(uint32_t)(h >> 32) & mask], 1u);
+    before += there;
+    most = max(most, there + 1u);
+  }
+  before = wave_reduce_sum(before);
+  for (int d = 32; d > 0; d >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, d, 64));
+  if (lane_id() == 0) {
+    if (before) atomicAdd(&out[0], before);
+    if (most > 1u) atomicMax(&out[1], (unsigned long long)most);
+  }
+}
+
+hipError_t launch_cell_crowding(const DeviceObjects &o, double inv_cell, const uint64_t *scen_off,
+                                uint32_t nscen, uint32_t *table, uint32_t mask, unsigned long long *out,
+                                hipStream_t s) {
+  const unsigned blocks = (unsigned)std::min<size_t>(512, (o.n + 255) / 256);
+  hipLaunchKernelGGL(k_cell_crowding, dim3(blocks), dim3(256), 0, s, o, inv_cell, scen_off, nscen, table, mask, out);
+  return hipGetLastError();
+}
+
 // The packed fields stand behind the arena's slots.
 __host__ __device__ __forceinline__ PackedObject *packed_objects(void *scratch, const TileParams &tp) {
   return reinterpret_cast<PackedObject *>(static_cast<char *>(scratch) + (size_t)tp.arena_cap * kArenaSlotBytes);

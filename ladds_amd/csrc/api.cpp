@@ -94,6 +94,9 @@ struct PipeBuffer {
 
 }  // namespace
 
+// How the objects share cells, by which the pair kernel is chosen (cell_shape).
+enum CellShape { kSparseCells, kCloudCells, kCrowdedCells };
+
 struct ladds_ctx {
   ladds_config cfg{};
   int form = kFormFp64;
@@ -164,10 +167,11 @@ struct ladds_ctx {
   size_t plane_order_alloc = 0;
 
   // Objects that share cells, as measure_crowding counted them: the mean number of others in an
-  // object's cell and the most in one cell.  Since then (follow_cells): detections, and the fewest
+  // object's cell, the most in one cell, and the choice.  Since then (follow_cells): detections, and the fewest
   // candidates of one (< 0: none yet).
   double crowding = 0.0;
   uint32_t fullest_cell = 0;
+  CellShape shape = kSparseCells;
   uint64_t detections = 0;
   double candidates = -1.0;
   bool tuning = false;  // ladds_autotune times shapes: none is changed beside it
@@ -338,7 +342,8 @@ hipError_t alloc_objects(DeviceObjects &o, size_t cap) {
 //            (clustered populations, one screening, split / FP64, sparse against crowded: 131,072
 //            objects with 9.5 conjunctions each 297 / 360 against 193 / 184 us, 524,288 with 40 each
 //            in FP64 4020 against 580), and where clouds alone make a mean of kCrowdedClouds
-//   clouds   the sorting kernel in the shape of a sparse population, from kCloud objects in one cell on
+//   clouds   the sorting kernel in the shape of a sparse population, from kCloud64 (kCloudSplit) objects in one
+//            cell on
 // A cloud of k fragments among n, one detection / a step of ladds_simulate, us, sparse against clouds
 // against crowded.  n 1,048,576, split: k 60 122 / 58, 130 / 69, 160 / 148; k 100 209 / 64, 161 / 77, 184
 // / 155; k 150 368 / 80, 204 / 86, 235 / 160; k 1000 11622 / 1487, 2771 / 493, 1267 / 408; FP64: k 100 223
@@ -346,11 +351,15 @@ hipError_t alloc_objects(DeviceObjects &o, size_t cap) {
 // 302.  n 65,521, split: k 100 236 / 36, 136 / 42, 112 / 44; k 600 6119 / 652, 1171 / 231, 769 / 201.
 constexpr double kCrowded = 2.0, kCrowdedClouds = 0.5;
 constexpr uint32_t kCloud64 = 128, kCloudSplit = 96;
-enum CellShape { kSparseCells, kCloudCells, kCrowdedCells };
 
-CellShape cell_shape(const ladds_ctx *ctx) {
-  const bool cloud = ctx->fullest_cell >= (ctx->form == kFormFp64 ? kCloud64 : kCloudSplit);
-  if (ctx->crowding >= kCrowded || (cloud && ctx->crowding >= kCrowdedClouds)) return kCrowdedCells;
+// The choice for the objects as they were counted.  A shape in use is left below 0.8 of its thresholds,
+// and a cloud's for the crowded one above 1.25 of them, so that a population near a threshold does not
+// change its shape again and again (the shape of 1,000,000 objects takes milliseconds).
+CellShape cell_shape(const ladds_ctx *ctx, CellShape was) {
+  const double stay = was == kSparseCells ? 1.0 : 0.8;
+  const double crowd = was == kCrowdedCells ? 0.8 : (was == kCloudCells ? 1.25 : 1.0);
+  const bool cloud = ctx->fullest_cell >= stay * (ctx->form == kFormFp64 ? kCloud64 : kCloudSplit);
+  if (ctx->crowding >= crowd * kCrowded || (cloud && ctx->crowding >= crowd * kCrowdedClouds)) return kCrowdedCells;
   return cloud ? kCloudCells : kSparseCells;
 }
 
@@ -388,7 +397,7 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   g.inv_cell_x = 1.0 / cell_x;
   // buckets two cells tall (wide): an object then scans two rows of the next plane (two
   // buckets of a row), not three
-  const bool crowded = cell_shape(ctx) == kCrowdedCells;
+  const bool crowded = ctx->shape == kCrowdedCells;
   const bool half_rows = tiles && (ctx->tune_rows == 2 || (ctx->tune_rows == 0 && crowded));
   const bool half_buckets = tiles && (ctx->tune_bcells == 2 || (ctx->tune_bcells == 0 && crowded));
   g.inv_cell_y = half_rows ? 0.5 * g.inv_cell : g.inv_cell;
@@ -624,7 +633,7 @@ int setup_grid(ladds_ctx *ctx, size_t n, const double *rx) {
   const bool chunks_chosen = (ctx->cfg.scan_chunks >= 1 && ctx->cfg.scan_chunks <= 32) ||
                              (ctx->tune_chunks >= 1 && ctx->tune_chunks <= 32);
   if (tiles && !plane_count.empty() && !(chunks_chosen && tp.nchunk > 1) && tp.persistent_groups == 0u &&
-      !valid_pair_threads(bs) && cell_shape(ctx) == kSparseCells) {
+      !valid_pair_threads(bs) && ctx->shape == kSparseCells) {
     // most records of a group of planes and the next one, with room for their drift
     auto group_max = [&](size_t group) {
       const size_t P = tp.nplanes;
@@ -761,12 +770,14 @@ int ensure_xbuf(ladds_ctx *ctx, size_t bytes) {
   return LADDS_OK;
 }
 
-// Counts the objects on the device by cell (side: the search radius; same scenario).  The table
+// Counts the objects on the device by cell (side: the search radius; same scenario) and chooses the
+// shape, coming from `was`.  The table
 // takes the place of the records, which every detection writes anew.
-int measure_crowding(ladds_ctx *ctx) {
+int measure_crowding(ladds_ctx *ctx, CellShape was = kSparseCells) {
   const size_t n = ctx->n;
   ctx->crowding = 0.0;
   ctx->fullest_cell = 0;
+  ctx->shape = kSparseCells;
   ctx->candidates = -1.0;
   ctx->detections = 0;
   if (n < 2 || ctx->variant != kVariantPlaneTiles) return LADDS_OK;
@@ -796,6 +807,7 @@ int measure_crowding(ladds_ctx *ctx) {
   const double by_chance = (double)(n - 1) / (double)words;  // cells that share an entry of the table
   ctx->crowding = std::max(0.0, 2.0 * (double)pairs / (double)n - by_chance);
   ctx->fullest_cell = (uint32_t)fullest;
+  ctx->shape = cell_shape(ctx, was);
   return LADDS_OK;
 }
 
@@ -814,14 +826,14 @@ int follow_cells(ladds_ctx *ctx, uint64_t candidates, uint64_t detections) {
   if (detections == 0 || ctx->n < 2 || ctx->variant != kVariantPlaneTiles || ctx->tuning) return LADDS_OK;
   constexpr uint64_t kCellsAgain = 64;
   constexpr double kFew = 2000.0;  // half the pairs of a cell of kCloudSplit
-  const CellShape shape = cell_shape(ctx);
+  const CellShape shape = ctx->shape;
   const double now = (double)candidates / (double)detections;
   ctx->detections += detections;
   ctx->candidates = ctx->candidates < 0.0 ? now : std::min(ctx->candidates, now);
   if (shape == kSparseCells ? now < 2.0 * ctx->candidates + kFew : ctx->detections < kCellsAgain) return LADDS_OK;
-  int rc = measure_crowding(ctx);
+  int rc = measure_crowding(ctx, shape);
   ctx->candidates = now;
-  if (rc == LADDS_OK && cell_shape(ctx) != shape) rc = reshape(ctx);
+  if (rc == LADDS_OK && ctx->shape != shape) rc = reshape(ctx);
   return rc;
 }
 
@@ -2267,7 +2279,7 @@ int ladds_simulate(ladds_ctx *ctx, uint64_t first_iteration, int nsteps, int tpc
   const bool use_graph = ctx->cfg.step_graph != 0 && tpcd == 1 && ctx->variant == kVariantPlaneTiles &&
                          !ctx->profiling && ctx->n > 0 && nsteps > 0;
   const bool use_overlap = !use_graph && ctx->variant == kVariantPlaneTiles && ctx->n > 0 && nsteps > 0 &&
-                           (ctx->n > kSerialObjects || tpcd > 2 || cell_shape(ctx) != kSparseCells);
+                           (ctx->n > kSerialObjects || tpcd > 2 || ctx->shape != kSparseCells);
   // The eager loop's first iteration runs on stream2 (overlapped_iteration's `fill`), and so
   // does what precedes it here (counter reset, spawn state, environments), after anything
   // still queued on the context's stream.

@@ -278,11 +278,17 @@ LADDS_API int ladds_delete_burnups(ladds_ctx *ctx, double min_altitude_km, size_
  * population-derived default), partition tile sizes (4096, 8192, 16384 objects) and the
  * pair kernel's LDS per plane pair (sized for 2-5 workgroups per CU, or automatic), one
  * dimension at a time (coordinate descent), and keep the fastest for this context.  Pair
- * results do not depend on the choice. */
+ * results do not depend on the choice.
+ * Where few objects share a cell, with one workgroup per plane and without persistent
+ * workgroups, a sparse pair kernel runs that sizes its own workgroups and LDS.  It follows
+ * cell_size_km, plane_width_km, tile_size, plane_order, ensemble_plane_objects and
+ * pair_streams; plane_bits, pair_threads, workgroups_per_cu, row_cells and bucket_cells are
+ * those of the kernel that takes over where cells hold clouds, and they are not searched
+ * while the sparse one runs (their defaults are returned). */
 typedef struct ladds_tuning {
   double cell_size_km;   /* chosen cell side [km]                               */
   int32_t plane_bits;    /* chosen log2 buckets per x-plane                     */
-  int32_t pair_threads;  /* chosen pair-kernel workgroup size                   */
+  int32_t pair_threads;  /* chosen pair-kernel workgroup size (sorting kernel)  */
   double scan_us;        /* device time of one detection with the choice [us]   */
                          /* (ladds_config.tune_simulate: wall time per step)    */
   double default_us;     /* the same for the untuned default [us]               */

@@ -456,7 +456,8 @@ class Engine:
 
     def autotune(self, dt_interp: float | None = None, repetitions: int = 3) -> dict:
         """Pick the plane-tile cell size, plane shape and pair workgroup size by timing the
-        conjunction scan on the current state (``ladds_autotune``)."""
+        conjunction scan on the current state (``ladds_autotune``; its declaration says which values
+        the sparse pair kernel follows)."""
         t = _abi.Tuning()
         dt = self.config.dt if dt_interp is None else dt_interp
         self._check(lib.ladds_autotune(self._h, float(dt), int(repetitions), C.byref(t)), "autotune")

@@ -1916,6 +1916,9 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
                  (int)ctx->tiles.nchunk, 0,
                  ctx->tiles.plane_order ? 1 : 0, 0, ctx->tiles.half_rows ? 2 : 1, ctx->tiles.half_buckets ? 2 : 1,
                  0, 0};
+  // The sparse pair kernel reads neither the workgroup size, LDS share and buckets nor their shape:
+  // where it runs at the current point, those dimensions would time the same kernel again.
+  bool sparse = ctx->tiles.sparse_threads != 0u;
   double default_us = 0.0;
   // the objective: one detection, or (ladds_config.tune_simulate) a burst of simulate steps
   auto measure = [&](double *t) {
@@ -1979,6 +1982,7 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
   order.push_back(9);
   for (const int dim : order) {
     if (dim == 8 && !ensemble) continue;
+    if (sparse && (dim == 1 || dim == 4 || dim == 6 || dim == 9 || dim == 11)) continue;
     std::vector<Cand> cands;
     std::array<int, 11> c{cur[0], cur[1], cur[2], cur[3], cur[4], cur[5], cur[6], cur[7], cur[8], cur[9], cur[10]};
     if (dim == 0)
@@ -2053,6 +2057,7 @@ int ladds_autotune(ladds_ctx *ctx, double dt_interp, int repetitions, ladds_tuni
         cur_cell = cand.cell;
         cur_fx = cand.fx;
         for (int k = 0; k < 11; ++k) cur[k] = cand.v[k];
+        sparse = ctx->tiles.sparse_threads != 0u;
       }
     }
   }

@@ -341,7 +341,8 @@ LADDS_API void *ladds_stream(ladds_ctx *ctx);
  * aom, bc_inv, cr, activity may be NULL (0, 0, 1, passive); g_rT / g_vT may be NULL (zero);
  * g_bc may be NULL (not computed).  The caller owns the checkpoint buffer
  * (ladds_adjoint_checkpoint_doubles() doubles) between forward and backward; the plan owns
- * a workspace, so calls on one plan must not overlap. */
+ * a workspace, so calls on one plan must not overlap.  It takes 336 bytes per object and 32
+ * steps, up to 256 MiB or 48 n checkpoint_every bytes, whichever is more, and at least 336 n. */
 typedef struct ladds_adjoint ladds_adjoint;
 typedef struct ladds_adjoint_config {
   uint64_t n;               /* objects                                      */

@@ -3,8 +3,10 @@
 A thin binding of the ``ladds_adjoint_*`` entry points of ``include/ladds_amd.h``,
 used only for this form: the forward pass and the hand-written adjoint both run as
 gfx950 kernels on torch's current HIP stream, on tensors torch owns.  There is no
-autograd tape through the propagation: ``YoshidaFlow.backward`` calls the adjoint
-kernel, which recomputes each checkpoint segment and sweeps it in reverse.
+autograd tape through the propagation: ``YoshidaFlow.backward`` makes two launches (or two for
+each group of chunks, where the trajectory's do not fit the plan's workspace).  The first runs
+every 32-step chunk again from its checkpoint, all chunks side by side, and stores its 6 x 7
+transition matrix; the second applies the transposed matrices from the last chunk to the first.
 
     plan = AdjointPlan(n=4096, nsteps=1440, dt=60.0, components=ALL_COMPONENTS)
     rT, vT = propagate(r0, v0, bc_inv, plan, aom=aom, cr=cr)   # (n, 3) float64 on cuda
@@ -41,7 +43,12 @@ if len(_hip_runtimes()) > 1:
 class AdjointPlan:
     """Per-(n, nsteps, dt, t0, components) state: the sub-step environments on the device
     and the backward workspace.  One plan serves any number of forward/backward pairs;
-    calls on one plan must not overlap (they share the workspace)."""
+    calls on one plan must not overlap (they share the workspace).
+
+    The workspace holds transition matrices, 336 bytes per object and 32-step chunk: those of the
+    whole trajectory up to 256 MiB (or up to the 48 bytes per object of a checkpoint segment's
+    states, where these are more), at least one chunk's and at most 1,024 chunks'; longer
+    trajectories go through it in groups."""
 
     def __init__(self, n: int, nsteps: int, dt: float, t0: float = 0.0, components: int = ALL_COMPONENTS,
                  checkpoint_every: int = 64, device: int = 0):

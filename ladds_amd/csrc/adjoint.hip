@@ -1,7 +1,9 @@
 // adjoint.hip -- hand-written adjoint of the FP64 Yoshida-4 propagation.
 //
-// Forward: the FP64 step of propagate.hip (the same acceleration<kFormFp64>), every step of
-// the trajectory in one launch, the state stored every K steps (checkpoints).
+// Forward: the FP64 step of propagate.hip, every step of the trajectory in one launch, the state
+// stored every K steps (checkpoints).  The force model stands here a second time, in four partial
+// accelerations that also give their derivatives (partial_*, the same terms and constants as
+// acceleration<kFormFp64>, fused and summed differently: the two agree to rounding).
 //
 // Backward: the gradient with respect to the initial state is a product of transition
 // matrices, lambda_c = Phi_c^T lambda_{c+1}, one for each chunk of kChunk steps.  A chunk's

@@ -185,7 +185,7 @@ struct ladds_ctx {
   double tune_fx = 0.0;  // plane width / cell size
   int tune_wgs = 0;      // pair-kernel workgroups per CU its LDS is sized for (0: automatic)
   int tune_order = 0;    // pair-kernel dispatch: 0 plane order, 1 heaviest runs of planes first
-  int tune_ens_plane = 0;  // ensembles: objects per x-plane the planes are sized for (0: 64)
+  int tune_ens_plane = 0;  // ensembles: objects per x-plane the planes are sized for (0: 256)
   int tune_rows = 0;       // bucket row height along y in cells: 2 or 1 (0: by the crowding)
   int tune_bcells = 0;     // bucket width along z in cells: 2 or 1 (0: by the crowding)
   int tune_persistent = 0; // 1: pair kernel as persistent workgroups with per-XCD queues

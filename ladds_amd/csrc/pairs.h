@@ -48,7 +48,7 @@ struct SoAObject {
 };
 
 // What the predicate reads of one object, side by side (k_pack_objects): one or two lines of the
-// cache where the object arrays take eleven.
+// cache where the object arrays take ten.
 struct alignas(16) PackedObject {
   double r[3], v[3];
   double rad;

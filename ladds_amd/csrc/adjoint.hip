@@ -109,6 +109,12 @@ __device__ __forceinline__ void keep_env(SubstepEnv<double> (&stage)[3], double 
   __builtin_amdgcn_wave_barrier();
 }
 
+// rsqrt64<true> with one instruction instead of three: scalar registers are free here (4,096 objects, a
+// day of 60 s steps: 2.58 ms, 2.61 with the other).
+__device__ __forceinline__ double rsqrt64_far(double x) {
+  return rsqrt64_step(fmin(x, 1.7976931348623157e308), __builtin_amdgcn_rsq(x));
+}
+
 // Derivatives of the acceleration at (r, v).
 struct Jacobian {
   double xx, xy, xz, yy, yz, zz;          // conservative part of da/dr (symmetric)
@@ -125,7 +131,7 @@ __device__ __forceinline__ void partial_field(double x, double y, double z, unsi
                                               double (&a)[3], Jacobian &o) {
 #pragma clang fp contract(on)
   const double r2 = x * x + y * y + z * z;
-  const double inv_r = rsqrt64<true>(r2);
+  const double inv_r = rsqrt64_far(r2);
   const double inv_r2 = inv_r * inv_r;
   const double inv_r3 = inv_r2 * inv_r;
   const double inv_r5 = inv_r3 * inv_r2;
@@ -204,7 +210,7 @@ __device__ __forceinline__ void partial_drag(double x, double y, double z, doubl
   const double inv_w = rsqrt64<false>(fmax(w2, 1e-290));
   const double wn = w2 * inv_w;  // 0 without wind
   const double r2 = x * x + y * y + z * z;
-  const double inv_r = rsqrt64<true>(r2);
+  const double inv_r = rsqrt64_far(r2);
   const double h = r2 * inv_r - kREarth;
   const AtmRow &row = atm_row(h, atm);
   const double inv_scale = row.inv_scale;
@@ -248,7 +254,7 @@ __device__ __forceinline__ void partial_central(double x, double y, double z, co
                                                 const double *indirect, bool gravity, double (&a)[3], Jacobian &o) {
 #pragma clang fp contract(on)
   const double dx = s[0] - x, dy = s[1] - y, dz = s[2] - z;
-  const double inv_d = rsqrt64<true>(dx * dx + dy * dy + dz * dz);
+  const double inv_d = rsqrt64_far(dx * dx + dy * dy + dz * dz);
   const double inv_d2 = inv_d * inv_d;
   const double f = k * (inv_d2 * inv_d);
   const double go = gravity ? 1.0 : 0.0;

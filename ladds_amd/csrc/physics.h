@@ -72,22 +72,29 @@ inline void fill_atm_table(AtmTable &t) {
   }
 }
 
-// 1/sqrt(x) of a positive x: the hardware's estimate (~2^-24) and one step of third order
-// (Householder's iteration), y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2, which leaves rounding
-// error only.  FAR: x may have overflowed and then gives 0 (its estimate; e is formed with a
-// finite x).  That is one instruction more: paid by every object it took 2% of 1,000 steps of
-// 250,007, so the propagation's paths for the usual models go without and leave the objects
-// beyond kFar to the general one.
+// 1/sqrt(x) of a positive x from the hardware's estimate y (~2^-24), one step of third order
+// (Householder's iteration): y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2, which leaves rounding
+// error only.
+__device__ __forceinline__ double rsqrt64_step(double x, double y) {
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+// FAR: x may have overflowed and then gives 0 (its estimate; e is formed with a finite x).  Paid
+// by every object that took 2% of 1,000 steps of 250,007, so the propagation's paths for the
+// usual models go without and leave the objects beyond kFar to the general one.  (On the high
+// word alone: a 64-bit constant would take scalar registers, which spill there and cost the
+// other paths of the split form 11 instructions a step.)
 template <bool FAR>
 __device__ __forceinline__ double rsqrt64(double x) {
   const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-(FAR ? fmin(x, 1.7976931348623157e308) : x) * y, y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
+  if (FAR) x = __hiloint2double((int)min((unsigned)__double2hiint(x), 0x7FEFFFFFu), __double2loint(x));
+  return rsqrt64_step(x, y);
 }
 
 // An object whose coordinates [km] sum up to less at the start of a launch does not come near the
 // overflow of its squared distances within it.
-constexpr double kFar = 1.0e140;
+constexpr double kFar = 0x1p465;  // ~1e140
 
 // a b + c with c a constant of the loop.  Written out because the compiler picks the two-address
 // form here and copies the constant into its destination first, one more instruction each.

@@ -148,10 +148,11 @@ __global__ __launch_bounds__(256) void k_propagate(PropagateArgs a) {
       acceleration<FORM, decltype(far)::value>(x, y, z, vx, vy, vz, p, m, e64, e32, atm, ax, ay, az);
     };
   };
-  const bool far = !(fabs(x) + fabs(y) + fabs(z) < kFar);
-  if (__ballot(mask != kAllBits || far) == 0ull)
+  const unsigned long long usual = __ballot(mask != kAllBits), j2 = __ballot(mask != (kKepBit | kJ2Bit)),
+                           far = __ballot(!(fabs(x) + fabs(y) + fabs(z) < kFar));
+  if ((usual | far) == 0ull)
     steps(with(kAllBits, std::false_type{}));
-  else if (__ballot(mask != (kKepBit | kJ2Bit) || far) == 0ull)
+  else if ((j2 | far) == 0ull)
     steps(with(kKepBit | kJ2Bit, std::false_type{}));
   else
     steps(with(mask, std::true_type{}));
